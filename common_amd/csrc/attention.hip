@@ -555,163 +555,204 @@ int pick_g(const AttnLaunch& a, hipStream_t s) {
 }
 
 // Causal attention of prompt rows in fp32, the attention of the fp32-weight prefill: row t of
-// sequence b (block (b*T + t, g)) attends cache rows 0..p0+t of KV head g for the G query heads of
-// the group, with the decode kernel's arithmetic (queries pre-scaled by log2(e)/sqrt(hd), online
-// softmax in base 2, 16-lane groups each streaming every 16th row in chunks of RU rows loaded
-// together, group states merged by lane swaps and through LDS).  The cache rows of the prompt are written beforehand (qk_prep), so every row
-// reads finished rows only.  q32: [B*T][heads*hd] normalised, rotated queries; caches fp32
-// [B][KV][S][hd]; out: [B*T][heads*hd].
-template <int HD, int G>
-__global__ __launch_bounds__(256) void attn_prefill_f32_kernel(const float* q32, const float* kcache,
-                                                                const float* vcache, float* out, int T, int p0,
-                                                                int S, int heads, int kv_heads) {
-    constexpr int EPL = HD / 16, NGR = 16, NWV = 4, RU = 4;
-    __shared__ __attribute__((aligned(16))) float red_acc[NWV][G][HD];
-    __shared__ float red_m[NWV][G], red_l[NWV][G];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = tid >> 4, gl = tid & 15;
-    const int r = blockIdx.x, g = blockIdx.y, b = r / T, t = r - b * T, n = p0 + t + 1;
-    const size_t head = ((size_t)b * kv_heads + g) * (size_t)S * HD;
-    const float* kc = kcache + head;
-    const float* vc = vcache + head;
-    auto dim_of = [&](int e) { return 16 * (e & ~3) + gl * 4 + (e & 3); };
-    const float c2 = 1.4426950408889634f / sqrtf((float)HD);
-    float qf[G][EPL];
-#pragma unroll
-    for (int h = 0; h < G; h++)
-#pragma unroll
-        for (int e = 0; e < EPL; e += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(q32 + (size_t)r * heads * HD + (size_t)(g * G + h) * HD +
-                                                              16 * e + gl * 4);
-            qf[h][e] = v.x * c2; qf[h][e + 1] = v.y * c2; qf[h][e + 2] = v.z * c2; qf[h][e + 3] = v.w * c2;
-        }
-    float m[G], l[G], acc[G][EPL];
-#pragma unroll
-    for (int h = 0; h < G; h++) {
-        m[h] = -INFINITY;
-        l[h] = 0.f;
-#pragma unroll
-        for (int e = 0; e < EPL; e++) acc[h][e] = 0.f;
-    }
-    auto load_row = [&](float (&dst)[EPL], const float* src, int row) {
-#pragma unroll
-        for (int e = 0; e < EPL; e += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(src + (size_t)row * HD + 16 * e + gl * 4);
-            dst[e] = v.x; dst[e + 1] = v.y; dst[e + 2] = v.z; dst[e + 3] = v.w;
-        }
-    };
-    // chunk c: rows c*NGR*RU + grp + NGR*j (j < RU) of each 16-lane group, loaded together (rows past
-    // n re-read row n-1 and score -inf); the next chunk is in flight while one is used
-    float ka[RU][EPL], va[RU][EPL], kb[RU][EPL], vb[RU][EPL];
-    auto load_chunk = [&](float (&kd)[RU][EPL], float (&vd)[RU][EPL], int c) {
-#pragma unroll
-        for (int j = 0; j < RU; j++) {
-            const int row = min(c * NGR * RU + grp + NGR * j, n - 1);
-            load_row(kd[j], kc, row);
-            load_row(vd[j], vc, row);
-        }
-    };
-    auto use_chunk = [&](const float (&kd)[RU][EPL], const float (&vd)[RU][EPL], int c) {
-        float sc[G][RU];
-#pragma unroll
-        for (int j = 0; j < RU; j++) {
-            const bool valid = c * NGR * RU + grp + NGR * j < n;
-#pragma unroll
-            for (int h = 0; h < G; h++) {
-                float d = 0.f;
-#pragma unroll
-                for (int e = 0; e < EPL; e++) d = fmaf(qf[h][e], kd[j][e], d);
-                d = row16_sum(d);
-                sc[h][j] = valid ? d : -INFINITY;
-            }
-        }
-#pragma unroll
-        for (int h = 0; h < G; h++) {
-            float mc = sc[h][0];
-#pragma unroll
-            for (int j = 1; j < RU; j++) mc = fmaxf(mc, sc[h][j]);
-            const float mn = fmaxf(m[h], mc);
-            if (mn == -INFINITY) continue;
-            const float alpha = (m[h] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[h] - mn);
-            l[h] *= alpha;
-#pragma unroll
-            for (int e = 0; e < EPL; e++) acc[h][e] *= alpha;
-#pragma unroll
-            for (int j = 0; j < RU; j++) {
-                const float pj = __builtin_amdgcn_exp2f(sc[h][j] - mn);
-                l[h] += pj;
-#pragma unroll
-                for (int e = 0; e < EPL; e++) acc[h][e] = fmaf(pj, vd[j][e], acc[h][e]);
-            }
-            m[h] = mn;
-        }
-    };
-    const int nch = (n + NGR * RU - 1) / (NGR * RU);
-    load_chunk(ka, va, 0);
-    for (int c = 0; c < nch; c += 2) {
-        if (c + 1 < nch) load_chunk(kb, vb, c + 1);
-        use_chunk(ka, va, c);
-        if (c + 1 >= nch) break;
-        if (c + 2 < nch) load_chunk(ka, va, c + 2);
-        use_chunk(kb, vb, c + 1);
-    }
-    auto merge_with = [&](auto partner) {
-#pragma unroll
-        for (int h = 0; h < G; h++) {
-            const float mo = partner(m[h]), lo = partner(l[h]);
-            const float mn = fmaxf(m[h], mo);
-            const float a = (m[h] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[h] - mn);
-            const float bo = (mo == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mo - mn);
-            l[h] = l[h] * a + lo * bo;
-#pragma unroll
-            for (int e = 0; e < EPL; e++) acc[h][e] = acc[h][e] * a + partner(acc[h][e]) * bo;
-            m[h] = mn;
-        }
-    };
-    merge_with([&](float v) { return xor16(v, lane); });
-    merge_with([&](float v) { return xor32(v, lane); });
-    if (lane < 16) {
-#pragma unroll
-        for (int h = 0; h < G; h++) {
-#pragma unroll
-            for (int e = 0; e < EPL; e++) red_acc[wave][h][dim_of(e)] = acc[h][e];
-            if (lane == 0) {
-                red_m[wave][h] = m[h];
-                red_l[wave][h] = l[h];
-            }
-        }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < G * HD; idx += 256) {
-        const int h = idx / HD, i = idx - h * HD;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < NWV; w++) M = fmaxf(M, red_m[w][h]);
-        float L = 0.f, o = 0.f;
-#pragma unroll
-        for (int w = 0; w < NWV; w++) {
-            const float wt = (red_m[w][h] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(red_m[w][h] - M);
-            L = fmaf(red_l[w][h], wt, L);
-            o = fmaf(red_acc[w][h][i], wt, o);
-        }
-        out[(size_t)r * heads * HD + (size_t)(g * G + h) * HD + i] = o / L;
-    }
-}
+// sequence b attends cache rows 0..p0+t of its KV head, fp32 products and sums throughout
+// (v_mfma_f32_32x32x2_f32), online softmax in base 2 with the queries pre-scaled by
+// log2(e)/sqrt(hd).  The cache rows of the prompt are written beforehand (qk_prep).
+// q32: [B*T][heads*hd] normalised, rotated queries; caches fp32 [B][KV][S][hd]; out: [B*T][heads*hd].
+//
+// Bound by the fp32 matrix rate: a 32-key x 32-query tile is hd MFMA instructions of 64 cycles
+// (hd 128: 8,192 cycles) against 32 KB of K and V, so the rows go straight from the caches into
+// registers and nothing but the queries needs LDS.  One block of four wavefronts takes 32 query rows
+// of one head; wavefront s takes key tiles s, s+4, ... (a causal block's work grows with its last
+// row: quarter-length chains in blocks taken heaviest first fill the CUs evenly, two blocks per CU),
+// and the four partial softmax states meet in LDS at the end, each wavefront folding a quarter of
+// the outputs.  Both products are computed transposed, so a lane owns one query (lanes l and l^32
+// hold the two halves of its scores) and the weights P feed the second product from the registers
+// the first one left them in:
+//   S^T (32 keys x 32 queries) = K . Q^T   contraction step (q, c): d = 8q + 4(l/32) + c, so a lane
+//                                          reads its key row and its query row 16 bytes at a time
+//   O^T (hd x 32 queries)     += V^T . P^T contraction step r: key (r/4)*8 + (l/32)*4 + r%4 (the
+//                                          result layout of S^T); output row i of tile j is dim
+//                                          NT*i + j, so one load per key row feeds every tile
+// K of the wavefront's next tile is loaded while P.V runs, V while the next Q.K runs.
+// 0.6B shape (16 heads, 8 KV heads, hd 128), 1,531 rows: 100 us (96 TFLOP/s of the causal half; the
+// matrix units are busy 60% of it, the rest is the uneven end of the causal blocks and each block's
+// start and merge) against 382 us for one block per (row, KV head) on the vector units, where each
+// row reads its whole context; 128 rows 10.9 against 11.4 us.
+struct PrefillAttnF32 {
+    const float *q32, *kcache, *vcache;
+    float* out;
+    int T, p0, S, heads, kv_heads, pairs, nq;  // pairs: B * kv_heads; nq: query tiles of 32 rows
+};
 
 template <int HD>
-int launch_prefill_f32_hd(const float* q32, const float* kc, const float* vc, float* out, int B, int T, int p0, int S,
-                          int heads, int kv_heads, hipStream_t st) {
-    const dim3 grid(B * T, kv_heads);
-    switch (heads / kv_heads) {
-        case 1: hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, 1>), grid, dim3(256), 0, st, q32, kc, vc, out, T, p0, S, heads, kv_heads); break;
-        case 2: hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, 2>), grid, dim3(256), 0, st, q32, kc, vc, out, T, p0, S, heads, kv_heads); break;
-        case 4: hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, 4>), grid, dim3(256), 0, st, q32, kc, vc, out, T, p0, S, heads, kv_heads); break;
-        case 8: hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, 8>), grid, dim3(256), 0, st, q32, kc, vc, out, T, p0, S, heads, kv_heads); break;
-        default:
-            ar_set_error("prefill attention: heads/kv_heads = %d not in {1,2,4,8}", heads / kv_heads);
-            return AR_HIP_ERR_INVALID;
+__global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32 p) {
+    typedef float floatx16 __attribute__((ext_vector_type(16)));
+    constexpr int KS = 4, NT = HD / 32, QROW = HD + 4;  // query row stride: conflict-free 16-byte reads
+    typedef float vrow __attribute__((ext_vector_type(NT)));
+    constexpr int STATE = NT * 16 + 2;                  // O^T, max and sum of a lane
+    constexpr int LDS_FLOATS = KS * STATE * 64 > 32 * QROW ? KS * STATE * 64 : 32 * QROW;
+    __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];
+
+    const int tid = threadIdx.x, lane = tid & 63, h2 = lane >> 5, lq = lane & 31;
+    const int slice = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // block -> (head, query tile), heaviest tiles first; the heads of one (sequence, KV head) on one
+    // XCD where the pair count allows, so its K and V stay in that XCD's L2
+    const int G = p.heads / p.kv_heads, units = p.pairs * G;
+    int pair, sub, qrank;
+    if (p.pairs % 8 == 0) {
+        const int slot = blockIdx.x >> 3, per = units >> 3, u = slot % per;
+        pair = (blockIdx.x & 7) + 8 * (u / G);
+        sub = u % G;
+        qrank = slot / per;
+    } else {
+        const int u = blockIdx.x % units;
+        pair = u / G;
+        sub = u % G;
+        qrank = blockIdx.x / units;
     }
-    AR_LAUNCH_CHECK();
-    return AR_HIP_OK;
+    const int b = pair / p.kv_heads, head = (pair - b * p.kv_heads) * G + sub;
+    const int row0 = (p.nq - 1 - qrank) * 32, myq = row0 + lq;
+    const float* kc = p.kcache + (size_t)pair * p.S * HD;
+    const float* vc = p.vcache + (size_t)pair * p.S * HD;
+    const int kend = p.p0 + min(row0 + 32, p.T);  // keys the block needs: 0 .. kend-1
+    const int ntiles = (kend + 31) / 32;
+
+    float4 kf[HD / 8];
+    vrow vf[16];
+    auto load_k = [&](int t) __attribute__((always_inline)) {
+        const unsigned at = (unsigned)min(32 * t + lq, kend - 1) * HD + 4 * h2;  // (32-bit: scalar base + offset)
+#pragma unroll
+        for (int q = 0; q < HD / 8; q++) kf[q] = *reinterpret_cast<const float4*>(kc + at + 8 * q);
+    };
+    auto load_v = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const unsigned key = min(32 * t + (r >> 2) * 8 + h2 * 4 + (r & 3), kend - 1);
+            vf[r] = *reinterpret_cast<const vrow*>(vc + key * HD + NT * lq);
+        }
+    };
+    // (past the wavefront's last tile the loads re-read the last key row: no branch around them, so the
+    // waits count exactly the loads they need)
+    const float c2 = 1.4426950408889634f / sqrtf((float)HD);
+    constexpr int QL = 32 * HD / 4 / 256;  // 16-byte query loads per thread, issued ahead of K and V
+    float4 qr[QL];
+#pragma unroll
+    for (int i = 0; i < QL; i++) {
+        const int r = (tid + 256 * i) / (HD / 4), c = tid % (HD / 4), t = min(row0 + r, p.T - 1);
+        qr[i] = *reinterpret_cast<const float4*>(p.q32 + ((size_t)b * p.T + t) * p.heads * HD + (size_t)head * HD + 4 * c);
+    }
+    load_k(slice);
+    load_v(slice);
+#pragma unroll
+    for (int i = 0; i < QL; i++) {
+        const int r = (tid + 256 * i) / (HD / 4), c = tid % (HD / 4);
+        *reinterpret_cast<float4*>(&lds[r * QROW + 4 * c]) =
+            make_float4(qr[i].x * c2, qr[i].y * c2, qr[i].z * c2, qr[i].w * c2);
+    }
+    // a barrier over LDS only: K and V stay in flight across it
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    floatx16 o[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[j][r] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    for (int t = slice; t < ntiles; t += KS) {
+        floatx16 s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = 0.f;
+        // (the query values of a step are read one step ahead and no further: registers)
+        const float* const qrow = &lds[lq * QROW + 4 * h2];
+        float4 qv = *reinterpret_cast<const float4*>(qrow);
+#pragma unroll
+        for (int q = 0; q < HD / 8; q++) {
+            float4 qn = qv;
+            if (q + 1 < HD / 8) qn = *reinterpret_cast<const float4*>(qrow + 8 * (q + 1));
+            __builtin_amdgcn_sched_barrier(0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].x, qv.x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].y, qv.y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].z, qv.z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].w, qv.w, s, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            qv = qn;
+        }
+        load_k(t + KS);
+        const int k0 = 32 * t;
+        if (k0 + 31 > p.p0 + row0) {  // tiles past the first row's own key (row0 + 31 >= T lies there too)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (k0 + (r >> 2) * 8 + h2 * 4 + (r & 3) > min(p.p0 + myq, kend - 1)) s[r] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
+        mx = max_xor32(mx);
+        if (__ballot(mx > m)) {
+            const float mn = fmaxf(m, mx);
+            const float alpha = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[j][r] *= alpha;
+            m = mn;
+        }
+        // a query whose keys in this wavefront's tiles are all masked so far keeps m = -inf: weights 0
+        const float mu = (m == -INFINITY) ? 0.f : m;
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[r] = __builtin_amdgcn_exp2f(s[r] - mu);
+            sum += s[r];
+        }
+        l += sum_xor32(sum);
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[r][j], s[r], o[j], 0, 0, 0);
+        load_v(t + KS);
+    }
+
+    __syncthreads();  // the queries are read: their LDS takes the states
+    float* const st = lds + lane;  // [slice][value][lane]
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) st[(slice * STATE + j * 16 + r) * 64] = o[j][r];
+    st[(slice * STATE + NT * 16) * 64] = m;
+    st[(slice * STATE + NT * 16 + 1) * 64] = l;
+    __syncthreads();
+    if (myq >= p.T) return;
+    // m is finite for slice 0 (key 0 is in its first tile); a slice without live keys keeps -inf
+    float ms[KS], wgt[KS], M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+        ms[k] = st[(k * STATE + NT * 16) * 64];
+        M = fmaxf(M, ms[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+        wgt[k] = (ms[k] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ms[k] - M);
+        L = fmaf(st[(k * STATE + NT * 16 + 1) * 64], wgt[k], L);
+    }
+    float* orow = p.out + ((size_t)b * p.T + myq) * p.heads * HD + (size_t)head * HD;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {  // result registers 4*slice + i: dims NT*(8*slice + 4*h2 + i) + j
+        vrow v;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            float a = 0.f;
+#pragma unroll
+            for (int k = 0; k < KS; k++) a = fmaf(st[(k * STATE + j * 16 + 4 * slice + i) * 64], wgt[k], a);
+            v[j] = a / L;
+        }
+        *reinterpret_cast<vrow*>(orow + NT * (8 * slice + 4 * h2 + i)) = v;
+    }
 }
 
 }  // namespace
@@ -722,10 +763,24 @@ int launch_attention_prefill_f32(const float* q32, const float* kcache, const fl
     AR_CHECK_ARG(heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "prefill attention: bad head counts");
     AR_CHECK_ARG(p0 >= 0 && p0 + T <= S, "prefill attention: rows %d..%d outside the %d-row cache", p0, p0 + T, S);
     AR_CHECK_ARG((long long)B * T <= 0x7fffffffLL && kv_heads <= 65535, "prefill attention: grid too large");
-    if (hd == 128) return launch_prefill_f32_hd<128>(q32, kcache, vcache, out, B, T, p0, S, heads, kv_heads, stream);
-    if (hd == 64) return launch_prefill_f32_hd<64>(q32, kcache, vcache, out, B, T, p0, S, heads, kv_heads, stream);
-    ar_set_error("prefill attention: head_dim %d not supported (64, 128)", hd);
-    return AR_HIP_ERR_INVALID;
+    const int G = heads / kv_heads;
+    AR_CHECK_ARG(G == 1 || G == 2 || G == 4 || G == 8, "prefill attention: heads/kv_heads = %d not in {1,2,4,8}", G);
+    PrefillAttnF32 p;
+    p.q32 = q32; p.kcache = kcache; p.vcache = vcache; p.out = out; p.T = T; p.p0 = p0; p.S = S; p.heads = heads;
+    p.kv_heads = kv_heads; p.pairs = B * kv_heads; p.nq = (T + 31) / 32;
+    const long long blocks = (long long)p.pairs * G * p.nq;
+    AR_CHECK_ARG(blocks <= 0x7fffffffLL, "prefill attention: grid too large");
+    const dim3 grid((unsigned)blocks);
+    if (hd == 128) {
+        hipLaunchKernelGGL(attn_prefill_f32_kernel<128>, grid, dim3(256), 0, stream, p);
+    } else if (hd == 64) {
+        hipLaunchKernelGGL(attn_prefill_f32_kernel<64>, grid, dim3(256), 0, stream, p);
+    } else {
+        ar_set_error("prefill attention: head_dim %d not supported (64, 128)", hd);
+        return AR_HIP_ERR_INVALID;
+    }
+    AR_LAUNCH_CHECK();
+    return AR_HIP_OK;
 }
 
 size_t attention_partial_floats(int batch, int heads, int max_splits, int hd) {

@@ -228,6 +228,28 @@ def test_prefill_fp32_weights_vs_oracle(ctx):
         np.testing.assert_array_equal(toks[b], rf[T:])
 
 
+@pytest.mark.parametrize("heads,kv,hd,T,batch", [(4, 4, 64, 1, 1), (4, 2, 64, 31, 2), (8, 2, 128, 33, 1),
+                                                 (8, 1, 64, 128, 1), (2, 2, 128, 130, 3), (16, 8, 128, 97, 1)])
+def test_prefill_fp32_attention_tiles_vs_oracle(ctx, heads, kv, hd, T, batch):
+    """The fp32 prompt attention at the edges of its 32-row tiles and four key slices (fewer tiles than
+    slices, one row past a tile, one tile past the slices), every heads-per-KV-head ratio and both
+    block orders.  fp32 sums of at most 130 terms over two layers stay within 1e-5 of the FP64 oracle
+    (130 * 2^-24 = 8e-6 worst case)."""
+    cfg = C.Qwen3Config(dim=128, hidden_dim=192, layer_count=2, head_count=heads, kv_head_count=kv, vocab_size=320,
+                        seq_len=T + 2, head_size=hd, max_batch=batch,
+                        qk_norm_mode=C.QK_NORM_PER_HEAD if T % 2 else C.QK_NORM_WHOLE)
+    sd = synthetic.state_dict(cfg, seed=T)
+    prompts = [synthetic.prompt_ids(T, cfg.vocab_size, seed=b) for b in range(batch)]
+    with Qwen3(cfg, sd, ctx) as m:
+        for b, p in enumerate(prompts):
+            m.model.set_prompt(p, seq=b)
+        lp = m.model.prefill(return_logits=True)
+        assert m.model.prefill_by_steps() == 0
+    for b, p in enumerate(prompts):
+        _, rl = oracle.OracleQwen3(cfg, sd, precision="fp64").generate(p, 1)
+        assert rel_err(lp[b], rl[T - 1]) <= 1e-5, rel_err(lp[b], rl[T - 1])
+
+
 def test_prefill_fp32_c3_prompt_vs_oracle(ctx):
     """BASELINE config 3 (Qwen3-0.6B shape, fp32, q_dim 2048 != dim): the 128-token prompt through
     the fp32 batched prefill, then 8 greedy steps, against the FP32 oracle's batched prompt pass
