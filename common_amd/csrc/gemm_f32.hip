@@ -5,9 +5,9 @@
 // LayerFeatures.dense (domain/graph/.../LayerFeatures.java:785-830) for prompt rows, which the
 // reference feeds one per step (engine/ml/.../AutoregressiveModel.java:295-308).
 //
-// The products are small in rows (a 128-token prompt), so a block of 32 (or 64) rows x 64 columns
-// splits its k range over KS groups of wavefronts (two wavefronts per SIMD at KS = 4) and each
-// wavefront stages its weight rows through LDS with direct copies one iteration ahead (see the kernel).
+// Bound by the fp32 matrix rate (157 TFLOP/s at 2.4 GHz; 137-150 over launches of 0.1-0.4 ms, whose
+// clock is lower).  One block per CU, in whole rounds of blocks, at the tile that wastes least of them
+// (see the launch rule).
 // Epilogues: STORE (+ bias), RESIDUAL (C += product), SWIGLU (C = (A.W2^T) * silu(A.W^T)), and
 // k-slices stored separately for the consumer to add in a fixed order.
 #include <atomic>
@@ -19,7 +19,7 @@ namespace {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f4 __attribute__((ext_vector_type(4)));  // (a native vector: stays in registers)
 
-constexpr int BK = 32;  // k granularity every launch accepts
+constexpr int BK = 32;  // k values of one tile, and the granularity every launch accepts
 
 struct Params {
     const float* A;   // [M][lda]
@@ -33,9 +33,8 @@ struct Params {
 // Output tile of block `bid`: consecutive blocks (one XCD takes every 8th) walk m fastest within
 // groups of 8 n-tiles, so blocks running together on an XCD share W column tiles in its L2.
 __device__ inline void tile_of(int bid, int mt, int nt, int* mi, int* ni) {
-    const int nblk = mt * nt;
-    int t = bid;
-    if (nblk % 8 == 0) t = (bid & 7) * (nblk >> 3) + (bid >> 3);
+    const int nblk = mt * nt, q = nblk >> 3, r = nblk & 7, xcd = bid & 7;
+    const int t = xcd * q + min(xcd, r) + (bid >> 3);
     *mi = t % mt;
     *ni = t / mt;
 }
@@ -48,214 +47,197 @@ __device__ inline void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// Block tile (32*WM) x 64: two column wavefronts x KS k-groups.  Wavefront (kg, wn) computes the WM
-// 32 x 32 output blocks of rows 0..32*WM-1 and columns wn*32..wn*32+31 over k-group kg's 32 k values
-// of every iteration (KS*32 per iteration); the KS partial sums meet in LDS at the end (added in
-// group order) and group 0 runs the epilogue.  Operands of one MFMA step: lanes 0-31 supply
-// k = 8q + c, lanes 32-63 k = 8q + 4 + c, for component c of the float4 each lane holds of chunk q, so
-// the 32x32x2 MFMA pairs equal k values of A and W.
-//  * W: every wavefront stages its own 32 rows x 32 k of each weight matrix through LDS with direct
-//    global -> LDS copies (`global_load_lds_dwordx4`: 64 lanes x 16 contiguous bytes, so the loads
-//    are coalesced; reading the rows straight into registers costs one 16-byte piece of 32 different
-//    rows per instruction: 12-20% slower at the 128-row prompt shapes), double-buffered one iteration
-//    ahead; the 16-byte chunk c of row r sits in slot c ^ (r & 7), so the eight lanes of one 16-byte
-//    read phase hit eight different bank groups.  Only the wavefront that copies a tile reads it: a
-//    vmcnt wait, no barrier.
-//  * A: the tile (32*WM rows x KS*32 k) is staged row-major in LDS (row stride KS*32 + 4 floats,
-//    conflict-free 16-byte reads), its next iteration prefetched in registers, swapped under two
-//    block barriers that wait for LDS only.
-// s_waitcnt immediates (vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at [15:14]): vmcnt v only
-constexpr int vm_imm(int v) { return (v & 15) | ((v >> 4) << 14) | (7 << 4) | (15 << 8); }
+// s_waitcnt immediates (vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at [15:14]): vmcnt v, lgkmcnt l
+constexpr int vm_imm(int v, int l = 15) { return (v & 15) | ((v >> 4) << 14) | (7 << 4) | (l << 8); }
 typedef __attribute__((address_space(3))) void lds_void;
-constexpr int BKG = 32;  // k values per k-group per iteration
 
-template <int WM, int KS, int EPI>
+// A block of four wavefronts takes 32*MB rows x 32*WN output columns (WN column wavefronts x KG = 4/WN
+// k-groups; SwiGLU blocks hold the gate and the up rows of their columns), one k-tile of 32 per
+// iteration out of ST LDS stages.  Operands of one MFMA step: lanes 0-31 supply k = 8q + c, lanes 32-63
+// k = 8q + 4 + c, for component c of the float4 each lane holds of chunk q, so the 32x32x2 MFMA pairs
+// equal k values of A and W.  Both operands go from global memory straight into LDS
+// (`global_load_lds_dwordx4`: 64 lanes x 16 contiguous bytes, coalesced, no staging registers), rows of
+// 8 chunks of 16 bytes, chunk c of row r in slot c ^ (r & 7), so the lanes of one 16-byte read phase hit
+// different bank groups.  The iteration's one barrier comes before its last MFMAs, once every fragment
+// of the tile is read: behind it the next tile is whole and this tile's stage is free for tile
+// ST ahead, and the last MFMAs cover the reads of the next tile's first fragments.  Each output is CH sums
+// (k-groups times k-tiles modulo CH / KG) added at the end: shorter chains of roundings.
+// The small tiles take eight or four stages: their products stream the weights, cold from HBM, and two
+// stages ran the 128-row products of a 0.6B layer in 28 (gate/up) and 20 us (the others) against 24 and
+// 13; the large tiles are as fast with two.
+// MFMA busy 86-88% of a block's cycles.  A second block on the CU does not raise that and makes the
+// last round uneven (both blocks of a pair end together, the leftover blocks pair up again on the CUs
+// that end first: 1,531 x 3,072 x 1,024 SwiGLU 164 us at one block per CU, 267 us at two), so a launch
+// asks for more than half of a CU's LDS.
+template <int MB, int WN, int CH, int EPI>
 struct F32Shape {
-    static constexpr int NW = (EPI == GEMV_EPI_SWIGLU) ? 2 : 1, WN = 2, NWAVE = WN * KS;
-    static constexpr int BKI = BKG * KS, SA = BKI + 4;
-    static constexpr int WT = 32 * BKG;                        // floats of one wavefront's tile of one matrix
-    static constexpr int W_FLOATS = 2 * NW * NWAVE * WT;       // double-buffered
-    static constexpr int RED_FLOATS = (KS - 1) * WN * NW * WM * 1024;
-    static constexpr int DYN = W_FLOATS > RED_FLOATS ? W_FLOATS : RED_FLOATS;
-    static constexpr int LDS_BYTES = (DYN + 32 * WM * SA) * 4;  // + the A tile
+    static constexpr int KG = 4 / WN, NB = EPI == GEMV_EPI_SWIGLU ? 2 : 1;
+    static constexpr int BM = 32 * MB, NOUT = 32 * WN, BN = NOUT * NB;  // output tile BM x NOUT, BN weight rows
+    static constexpr int STAGE = (BM + BN) * BK;               // floats of one stage
+    // stages: two, or for the small tiles (CH 4) eight or four of them, up to 152 KB
+    static constexpr int ST = CH <= 2 ? 2 : 8 * STAGE <= 38 * 1024 ? 8 : 4;
+    static constexpr int RED = KG > 1 ? WN * MB * NB * 1024 : 0;  // the second k-group's sums
+    static constexpr int USED = (ST * STAGE > RED ? ST * STAGE : RED) * 4;
+    // more than half of a CU's 160 KB: one block per CU
+    static constexpr int LDS_BYTES = USED > 82 * 1024 ? USED : 82 * 1024;
 };
 
-template <int WM, int KS, int EPI>
-__global__ __launch_bounds__(128 * KS) void gemm_f32_kernel(Params p, int mt, int nt) {
-    using Sh = F32Shape<WM, KS, EPI>;
-    constexpr int NW = Sh::NW, WN = Sh::WN, NWAVE = Sh::NWAVE;
-    constexpr int BM = 32 * WM, NT = 64 * NWAVE;
-    constexpr int BKI = Sh::BKI, SA = Sh::SA, WT = Sh::WT;
-    constexpr int QG = BKG / 8;            // float4 chunks per lane per iteration
-    constexpr int AL = BM * BKI / 4 / NT;  // float4 A loads per thread per iteration
-    static_assert(AL >= 1 && (BM * BKI / 4) % NT == 0, "tile / thread shape");
+template <int MB, int WN, int CH, int EPI>
+__global__ __launch_bounds__(256, 1) void gemm_f32_kernel(Params p, int mt, int nt) {
+    using Sh = F32Shape<MB, WN, CH, EPI>;
+    constexpr int ST = Sh::ST;
+    constexpr int NB = Sh::NB, KG = Sh::KG, NA = CH / KG;  // NA sums per output and wavefront
+    constexpr int NQ = BK / 8 / KG;                       // float4 chunks per lane of a k-tile
+    constexpr int CP = (Sh::BM + Sh::BN) / 32;            // copies (8 rows each) per wavefront and stage
     extern __shared__ __attribute__((aligned(1024))) float dsm[];
-    float* const sw = dsm;            // [2][NW][NWAVE][32 rows x BKG]; the k-group reduction after the loop
-    float* const sa = dsm + Sh::DYN;  // A tile
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kg = wave / WN, wn = wave - kg * WN;
-    const int tiles = mt * nt;
-    const int ks = blockIdx.x / tiles;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / WN, wn = wave % WN;
+    const int tiles = mt * nt, ks = blockIdx.x / tiles;
     int mi, ni;
     tile_of(blockIdx.x - ks * tiles, mt, nt, &mi, &ni);
-    const int m0 = mi * BM, n0 = ni * 64;
-    const int kper = p.K / p.ksplit, kbase = ks * kper, nit = kper / BKI;
-    const int h = lane >> 5, l32 = lane & 31;
+    const int m0 = mi * Sh::BM, n0 = ni * Sh::NOUT;
+    const int kper = p.K / p.ksplit, kbase = ks * kper, nit = kper / BK;
 
-    f4 ra[AL];
-    auto load_a = [&](int it) __attribute__((always_inline)) {
-        const int k0 = kbase + it * BKI;
-#pragma unroll
-        for (int i = 0; i < AL; i++) {
-            const int e = tid + i * NT, r = e / (BKI / 4), c = e - r * (BKI / 4);
-            const int row = min(m0 + r, p.M - 1);  // rows past M re-read the last row (never stored)
-            ra[i] = *reinterpret_cast<const f4*>(p.A + (size_t)row * p.lda + k0 + 4 * c);
-        }
-    };
-    auto store_a = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < AL; i++) {
-            const int e = tid + i * NT, r = e / (BKI / 4), c = e - r * (BKI / 4);
-            *reinterpret_cast<f4*>(&sa[r * SA + 4 * c]) = ra[i];
-        }
-    };
-    // copy i of matrix x fills rows 8i .. 8i+7 of the wavefront's 32 weight rows: lane l writes slot
-    // l % 8 of row 8i + l / 8, i.e. fetches chunk (l % 8) ^ (row & 7); the LDS destination (M0) is
-    // uniform over the wavefront
-    const float* wsrc[NW];
+    // a stage holds the A rows, then the W rows (gate, then up); copy i of this wavefront fills rows
+    // 8*(4i + wave) .. +7, lane l slot l % 8 of row l / 8 (rows past M re-read the last row)
     const int drow = lane >> 3, dslot = lane & 7;
+    const float* src[CP];
 #pragma unroll
-    for (int x = 0; x < NW; x++) wsrc[x] = (x ? p.W2 : p.W) + (size_t)(n0 + wn * 32) * p.ldw + kbase + kg * BKG;
-    auto copy_w = [&](int it, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < NW; x++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = 8 * i + drow;
-                const float* g = wsrc[x] + (size_t)r * p.ldw + it * BKI + 4 * (dslot ^ (r & 7));
-                float* d = sw + ((buf * NW + x) * NWAVE + wave) * WT + i * 256;
-                __builtin_amdgcn_global_load_lds((const void*)g, (lds_void*)d, 16, 0, 0);
-            }
-    };
-    f4 wr[NW][QG];
-    auto read_w = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < NW; x++)
-#pragma unroll
-            for (int q = 0; q < QG; q++) {
-                const int c = 2 * q + h;
-                wr[x][q] = *reinterpret_cast<const f4*>(sw + ((buf * NW + x) * NWAVE + wave) * WT + l32 * BKG +
-                                                        4 * (c ^ (l32 & 7)));
-            }
-    };
-
-    floatx16 acc[NW][WM];
-#pragma unroll
-    for (int x = 0; x < NW; x++)
-#pragma unroll
-        for (int i = 0; i < WM; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[x][i][r] = 0.f;
-    auto compute = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int q = 0; q < QG; q++)
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-                const f4 a = *reinterpret_cast<const f4*>(&sa[(i * 32 + l32) * SA + kg * BKG + 8 * q + 4 * h]);
-#pragma unroll
-                for (int x = 0; x < NW; x++) {
-                    acc[x][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, wr[x][q].x, acc[x][i], 0, 0, 0);
-                    acc[x][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, wr[x][q].y, acc[x][i], 0, 0, 0);
-                    acc[x][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, wr[x][q].z, acc[x][i], 0, 0, 0);
-                    acc[x][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, wr[x][q].w, acc[x][i], 0, 0, 0);
-                }
-            }
-    };
-
-    // iteration it: the A tile `it` in LDS, this wavefront's W tile `it` in buffer it & 1; the next
-    // iteration's A rows (registers) and W copies (the other buffer, last read by this wavefront in
-    // the previous iteration) are issued first (the last iteration re-copies its own tile: the
-    // counts of every wait stay static)
-    load_a(0);
-    copy_w(0, 0);
-    __builtin_amdgcn_s_waitcnt(vm_imm(0));
-    store_a();
-    lds_barrier();
-    for (int it = 0; it < nit; it++) {
-        load_a(min(it + 1, nit - 1));
-        copy_w(min(it + 1, nit - 1), (it + 1) & 1);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(vm_imm(AL + 4 * NW));  // this wavefront's W tile `it` has landed
-        asm volatile("" ::: "memory");
-        read_w(it & 1);
-        compute();
-        lds_barrier();
-        if (it + 1 >= nit) break;
-        __builtin_amdgcn_s_waitcnt(vm_imm(4 * NW));  // the A rows have landed (the W copies may still fly)
-        store_a();
-        lds_barrier();
+    for (int i = 0; i < CP; i++) {
+        const int r = 8 * (4 * i + wave) + drow, w = r - Sh::BM;
+        const float* row = r < Sh::BM ? p.A + (size_t)min(m0 + r, p.M - 1) * p.lda
+                           : w < Sh::NOUT ? p.W + (size_t)(n0 + w) * p.ldw
+                                          : p.W2 + (size_t)(n0 + w - Sh::NOUT) * p.ldw;
+        src[i] = row + kbase + 4 * (dslot ^ (r & 7));
     }
-    __builtin_amdgcn_s_waitcnt(vm_imm(0));  // no copy in flight when the buffers are reused below
-    lds_barrier();
+    auto copy = [&](int it, int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < CP; i++)
+            __builtin_amdgcn_global_load_lds((const void*)(src[i] + it * BK),
+                                             (lds_void*)(dsm + st * Sh::STAGE + (4 * i + wave) * 256), 16, 0, 0);
+    };
 
-    // k-groups 1..KS-1 hand their sums to group 0, which adds them in group order
-    if constexpr (KS > 1) {
+    floatx16 acc[NA][MB][NB];
+#pragma unroll
+    for (int k = 0; k < NA; k++)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[k][i][j][r] = 0.f;
+    f4 a[2][MB], w[2][NB];
+    auto read = [&](int st, int q) __attribute__((always_inline)) {
+        const float* const row = dsm + st * Sh::STAGE + l32 * BK + 4 * ((2 * (kg * NQ + q) + h) ^ (l32 & 7));
+#pragma unroll
+        for (int i = 0; i < MB; i++) a[q & 1][i] = *reinterpret_cast<const f4*>(row + 32 * i * BK);
+#pragma unroll
+        for (int j = 0; j < NB; j++) w[q & 1][j] = *reinterpret_cast<const f4*>(row + (Sh::BM + j * Sh::NOUT + 32 * wn) * BK);
+    };
+    auto step = [&](int it, int u) __attribute__((always_inline)) {  // u: it modulo U
+        const int st = u % ST;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            if (q + 1 < NQ) {
+                read(st, q + 1);
+            } else {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(vm_imm((ST - 2) * CP, 0));  // tile it + 1 copied, tile `it` read
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                read((st + 1) % ST, 0);
+                copy(min(it + ST, nit - 1), st);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < MB; i++)
+#pragma unroll
+                    for (int j = 0; j < NB; j++)
+                        acc[u % NA][i][j] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(a[q & 1][i][e], w[q & 1][j][e], acc[u % NA][i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // (past the last tile the copies re-read it into a stage nobody reads)
+#pragma unroll
+    for (int i = 0; i < ST; i++) copy(min(i, nit - 1), i);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vm_imm((ST - 1) * CP));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    constexpr int U = ST > NA ? ST : NA;  // tiles per turn: the stage and the sum are compile-time indexes
+    int it = 0;
+    for (; it + U <= nit; it += U)
+#pragma unroll
+        for (int u = 0; u < U; u++) step(it + u, u);
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+        if (it + u < nit) step(it + u, u);
+    __builtin_amdgcn_s_waitcnt(vm_imm(0, 0));
+    __builtin_amdgcn_s_barrier();  // no copy and no read in flight
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int k = 1; k < NA; k++)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[0][i][j][r] += acc[k][i][j][r];
+    if constexpr (KG > 1) {  // the second k-group hands its sums over
+        float* const red = dsm + wn * (MB * NB * 1024) + lane;
         if (kg > 0) {
 #pragma unroll
-            for (int x = 0; x < NW; x++)
+            for (int i = 0; i < MB; i++)
 #pragma unroll
-                for (int i = 0; i < WM; i++) {
-                    float* d = &dsm[((((kg - 1) * WN + wn) * NW + x) * WM + i) * 1024 + lane];
+                for (int j = 0; j < NB; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) d[r * 64] = acc[x][i][r];
-                }
+                    for (int r = 0; r < 16; r++) red[((i * NB + j) * 16 + r) * 64] = acc[0][i][j][r];
         }
         lds_barrier();
         if (kg > 0) return;
 #pragma unroll
-        for (int g = 1; g < KS; g++)
+        for (int i = 0; i < MB; i++)
 #pragma unroll
-            for (int x = 0; x < NW; x++)
+            for (int j = 0; j < NB; j++)
 #pragma unroll
-                for (int i = 0; i < WM; i++) {
-                    const float* s = &dsm[((((g - 1) * WN + wn) * NW + x) * WM + i) * 1024 + lane];
-#pragma unroll
-                    for (int r = 0; r < 16; r++) acc[x][i][r] += s[r * 64];
-                }
+                for (int r = 0; r < 16; r++) acc[0][i][j][r] += red[((i * NB + j) * 16 + r) * 64];
     }
 
-    // output block (i) of this wave: lane holds column (lane & 31), rows (r>>2)*8 + (lane>>5)*4 + (r&3)
-    const int col = n0 + wn * 32 + l32;
-    float* const Cs = p.C + (size_t)ks * p.M * p.ldc;
+    // output block: lane holds column (lane & 31), rows (r>>2)*8 + (lane>>5)*4 + (r&3)
+    const int col = n0 + 32 * wn + l32;
+    const float bias = EPI == GEMV_EPI_STORE && p.bias ? p.bias[col] : 0.f;
+    float* const Cs = p.C + (size_t)ks * p.M * p.ldc + col;
 #pragma unroll
-    for (int i = 0; i < WM; i++)
+    for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const int row = m0 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+            const int row = m0 + 32 * i + (r >> 2) * 8 + h * 4 + (r & 3);
             if (row >= p.M) continue;
-            float* c = Cs + (size_t)row * p.ldc + col;
+            float* c = Cs + (size_t)row * p.ldc;
             if (EPI == GEMV_EPI_STORE) {
-                *c = p.bias ? acc[0][i][r] + p.bias[col] : acc[0][i][r];
+                *c = p.bias ? acc[0][i][0][r] + bias : acc[0][i][0][r];
             } else if (EPI == GEMV_EPI_RESIDUAL) {
-                *c = *c + acc[0][i][r];
+                *c = *c + acc[0][i][0][r];
             } else {
-                const float g = acc[0][i][r], u = acc[NW - 1][i][r];
+                const float g = acc[0][i][0][r], u = acc[0][i][NB - 1][r];
                 const float sg = 1.0f / (expf(-g) + 1.0f);
                 *c = u * (g * sg);
             }
         }
 }
 
-template <int WM, int KS, int EPI>
+template <int MB, int WN, int CH, int EPI>
 int launch_t(const Params& p, hipStream_t st) {
-    using Sh = F32Shape<WM, KS, EPI>;
+    using Sh = F32Shape<MB, WN, CH, EPI>;
     static_assert(Sh::LDS_BYTES <= 160 * 1024, "LDS");
-    const int mt = (p.M + 32 * WM - 1) / (32 * WM), nt = p.N / 64;
+    const int mt = (p.M + Sh::BM - 1) / Sh::BM, nt = p.N / Sh::NOUT;
     const long long blocks = (long long)mt * nt * p.ksplit;
     AR_CHECK_ARG(blocks <= 0x7fffffffLL, "GEMM f32: too many blocks");
-    auto kern = gemm_f32_kernel<WM, KS, EPI>;
+    auto kern = gemm_f32_kernel<MB, WN, CH, EPI>;
     // more than 64 KB of dynamic LDS needs the per-kernel opt-in, once per device
     static std::atomic<bool> attr_set[kMaxDevices];
     const int slot = ar_device_slot(st);
@@ -263,23 +245,62 @@ int launch_t(const Params& p, hipStream_t st) {
         AR_HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Sh::LDS_BYTES));
         if (slot >= 0) attr_set[slot].store(true, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(128 * KS), Sh::LDS_BYTES, st, p, mt, nt);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), Sh::LDS_BYTES, st, p, mt, nt);
     AR_LAUNCH_CHECK();
     return AR_HIP_OK;
 }
 
-// 64-row tiles once there are enough rows to fill the CUs with them (the W registers then feed two
-// output blocks), else 32-row tiles; as many k-groups as the k-slice divides into
+// The tile with the least time over whole rounds of one block per CU: a round of 32*MB x 32*WN tiles
+// takes their MFMA cycles over 0.87 and some 2,500 cycles of start, k-group fold and stores.  Measured
+// (us; the forms before this kernel, then the chosen tile against the next best): 1,531 x 4,096 x 1,024
+// 118, 96 x 128 in two rounds 111, 128 x 128 in two 145; 1,531 x 1,024 x 3,072 113, 96 x 64 in one round
+// 85, 64 x 128 in one 102; 1,531 x 3,072 x 1,024 SwiGLU 218, 96 x 64 in three 164, 64 x 64 in five 199;
+// 2,048 x 6,144 x 2,048 SwiGLU 954, 128 x 64 in six 799.  Below 512 rows the sums stay in four chains
+// (as many roundings as the 32-row form with four k-groups that ran there), which leaves registers for
+// at most 64 rows: 256 x 3,072 x 1,024 SwiGLU 48 -> 40, 128 x 4,096 x 1,024 15.6 -> 14.6 (us, repeated
+// calls on the same operands).
 template <int EPI>
-int launch_epi(const Params& p, hipStream_t st) {
-    const int kper = p.K / p.ksplit;
-    if (p.M >= 512) {
-        if (kper % 64 == 0) return launch_t<2, 2, EPI>(p, st);
-        return launch_t<2, 1, EPI>(p, st);
+int launch_epi(const Params& p, hipStream_t st, int cus) {
+    constexpr bool SW = EPI == GEMV_EPI_SWIGLU;
+    const int kper = p.K / p.ksplit, max_mb = p.M >= 512 ? 4 : 2;
+    int mb = 1, wn = 2;
+    double best = 0;
+    for (int w = 2; w <= (SW ? 2 : 4); w += 2)
+        for (int b = 1; b <= max_mb; b++) {
+            if (p.N % (32 * w)) continue;
+            const long long blocks = (long long)((p.M + 32 * b - 1) / (32 * b)) * (p.N / (32 * w)) * p.ksplit;
+            const double rounds = (double)((blocks + cus - 1) / cus);
+            const double cost = rounds * (8.0 * b * w * (SW ? 2 : 1) * kper / 0.87 + 2500.0);
+            if (best == 0 || cost < best) {
+                best = cost;
+                mb = b;
+                wn = w;
+            }
+        }
+#define AR_F32_TILE(MBV, WNV, CHV) \
+    if (mb == MBV && wn == WNV) return launch_t<MBV, WNV, CHV, EPI>(p, st)
+    if (p.M < 512) {
+        AR_F32_TILE(1, 2, 4);
+        AR_F32_TILE(2, 2, 4);
+        if constexpr (!SW) {
+            AR_F32_TILE(1, 4, 4);
+            AR_F32_TILE(2, 4, 4);
+        }
+    } else {
+        AR_F32_TILE(1, 2, 2);
+        AR_F32_TILE(2, 2, 2);
+        AR_F32_TILE(3, 2, 2);
+        AR_F32_TILE(4, 2, 2);
+        if constexpr (!SW) {
+            AR_F32_TILE(1, 4, 2);
+            AR_F32_TILE(2, 4, 2);
+            AR_F32_TILE(3, 4, 2);
+            AR_F32_TILE(4, 4, 2);
+        }
     }
-    if (kper % 128 == 0) return launch_t<1, 4, EPI>(p, st);
-    if (kper % 64 == 0) return launch_t<1, 2, EPI>(p, st);
-    return launch_t<1, 1, EPI>(p, st);
+#undef AR_F32_TILE
+    ar_set_error("GEMM f32: no tile for %d x %d", p.M, p.N);
+    return AR_HIP_ERR_INVALID;
 }
 
 }  // namespace
@@ -307,12 +328,13 @@ int launch_gemm_f32(const GemmF32Launch& a, hipStream_t stream) {
     Params p;
     p.A = a.A; p.W = a.W; p.W2 = a.W2; p.bias = a.bias; p.C = a.C;
     p.M = a.M; p.N = a.N; p.K = a.K; p.lda = a.lda; p.ldw = a.ldw; p.ldc = a.ldc; p.ksplit = a.ksplit;
+    const int cus = ar_device_cus(stream);
     switch (a.epilogue) {
-        case GEMV_EPI_STORE: return launch_epi<GEMV_EPI_STORE>(p, stream);
-        case GEMV_EPI_RESIDUAL: return launch_epi<GEMV_EPI_RESIDUAL>(p, stream);
+        case GEMV_EPI_STORE: return launch_epi<GEMV_EPI_STORE>(p, stream, cus);
+        case GEMV_EPI_RESIDUAL: return launch_epi<GEMV_EPI_RESIDUAL>(p, stream, cus);
         case GEMV_EPI_SWIGLU:
             AR_CHECK_ARG(a.W2, "GEMM f32: SwiGLU needs W2");
-            return launch_epi<GEMV_EPI_SWIGLU>(p, stream);
+            return launch_epi<GEMV_EPI_SWIGLU>(p, stream, cus);
     }
     ar_set_error("GEMM f32: unsupported epilogue %d", a.epilogue);
     return AR_HIP_ERR_INVALID;

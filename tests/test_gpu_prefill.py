@@ -181,11 +181,17 @@ def test_prefill_matches_sequential_decode_and_oracle(ctx, per_head, batch, back
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 64, 32), (16, 512, 256), (33, 64, 96), (40, 128, 768), (100, 768, 1024),
-                                   (128, 4096, 1024), (600, 1024, 3072), (520, 128, 160)])
+                                   (128, 4096, 1024), (600, 1024, 3072), (520, 128, 160),
+                                   # the tiles of the launch rule on 256 CUs, ragged M: below 512 rows
+                                   # 32 x 128, 64 x 64, 64 x 128; from 512 rows 32 x 64, 32 x 128, 64 x 64,
+                                   # 64 x 128, 96 x 64, 96 x 128, 128 x 64, 128 x 128
+                                   (152, 6528, 32), (39, 8960, 64), (476, 2560, 96), (663, 576, 64),
+                                   (777, 1280, 1344), (814, 1152, 32), (1185, 1664, 800), (533, 4800, 32),
+                                   (846, 3072, 96), (1411, 2368, 64), (3308, 1024, 32)])
 def test_gemm_f32_vs_float64(ctx, M, N, K):
-    """fp32 MFMA projection (ar_hip_gemm_f32): 32- and 64-row tiles, ragged M, 1 / 2 / 4 k-groups per
-    block with odd and even iteration counts, all three epilogues, against float64 products of the
-    same fp32 operands (1e-5 relative)."""
+    """fp32 MFMA projection (ar_hip_gemm_f32): every tile of the launch rule, ragged M, one to many
+    k-tiles of 32 (odd and even counts), all three epilogues, against float64 products of the same fp32
+    operands (1e-5 relative)."""
     r = np.random.default_rng(M + N + K)
     A = r.standard_normal((M, K)).astype(np.float32)
     W = (r.standard_normal((N, K)) * 0.05).astype(np.float32)
