@@ -14,14 +14,19 @@
 // sorted in descending order (ties in index order: Arrays.sort is stable) whose running sum
 // reaches top_p.  With p* the smallest kept value, that is every value > p* plus the first c
 // (by index) of the values == p*; p* is the largest key t with sum(p >= t) >= top_p.  It is found
-// by a radix descent over the 64-bit patterns of the probabilities (non-negative doubles order as
-// their bit patterns): 8 passes of 8-bit digits.  Each pass is one kernel: every chunk builds its
-// histogram of (count, sum) in LDS and adds it into the row's histogram with device-scope integer
-// atomics; the last chunk to finish (an arrival counter) picks the digit and clears the row's
-// histogram and counter for the next pass.  Bucket sums are 2^-60 fixed point in u64, so the
-// atomics are exact and associative (the result does not depend on arrival order); the kept set
-// agrees with the reference's sequential double sums except when top_p lies within ~1e-13 of a
-// partial sum.
+// on the 64-bit patterns of the probabilities (non-negative doubles order as their bit patterns):
+//  * one pass over the row adds the values into 1,024 buckets by exponent and the first four mantissa
+//    bits (64 octaves below 1; what lies lower is below the fixed point's unit and never holds p*), LDS
+//    per chunk, then the row's buckets with device-scope atomics; the last chunk to finish (an arrival
+//    counter) picks the bucket whose range holds p* and clears the row's buckets for the next draw;
+//  * one pass copies that bucket's values, in index order, and sums what lies above it per chunk;
+//  * the block that draws finishes the search on the copied values alone (a radix descent over the
+//    remaining 48 bits, 8 at a time, ending early once one value is left).
+// 8 x 151,936 values: 55 us a draw (draw 20, buckets 14, exponentials 11, copy 6.5, maximum 4: launches and
+// the serial chain of the drawing block, not the 4.9 MB of logits), against 124 with eight 8-bit passes over the whole row, whose
+// first digits separate next to nothing.  Bucket sums are 2^-60 fixed point in u64, so the atomics are
+// exact and associative (the result does not depend on arrival order); the kept set agrees with the
+// reference's sequential double sums except when top_p lies within ~1e-13 of a partial sum.
 //
 // The draw mirrors the reference's loop `cumulative += probs[i]; if (r < cumulative) return i`:
 // chunk masses locate the chunk whose interval holds r, then per-thread sums of contiguous index
@@ -35,26 +40,28 @@ namespace {
 constexpr int kBlocks = 64;   // chunks per row (one wavefront of partials)
 constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
+constexpr int kBins = 1024;   // buckets of the nucleus search (one per thread of the block that picks)
+constexpr int kCandLds = 4096;  // bucket values the drawing block holds in LDS
 constexpr double kFix = 1152921504606846976.0;     // 2^60
 constexpr double kEps64 = 2.220446049250313e-16;   // FP64 machine epsilon (Precision.java:110-121)
 
 struct Ws {
-    double* buf;                // [rows][V] exp values
+    double* buf;                // [rows][V] exp values; probabilities once the nucleus search began
     double* pmax;               // [rows][kBlocks]
     double* psum;
     double* pemax;
     double* psum2;
     double* pmass;
-    unsigned* hcnt;             // [rows][kBlocks][256] per-chunk counts of the last pass
-    unsigned* gcnt;             // [rows][256] row histogram of the current pass (zero between passes)
-    unsigned long long* gsum;   // [rows][256]
-    unsigned* arrived;          // [rows] chunks done with the current pass (zero between passes)
-    unsigned long long* sel;    // [rows][8]: prefix, above, done, take
+    unsigned long long* gsum;   // [rows][kBins] fixed-point bucket sums of the row (zero between draws)
+    unsigned* arrived;          // [rows] chunks done with the bucket pass (zero between draws)
+    unsigned long long* sel;    // [rows][2]: bucket of p* (or -1: everything is kept), fixed-point sum above it
+    unsigned long long* cand;   // [rows][V] bit patterns of the bucket's values, each chunk's at its own start
+    unsigned* ncand;            // [rows][kBlocks]
 };
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The zero-initialised part (gcnt, gsum, arrived) comes first so that it can be cleared once.
+// The zero-initialised part (gsum, arrived) comes first so that it can be cleared once.
 Ws carve(void* base, int rows, int V, size_t* total, size_t* zero_bytes) {
     Ws w{};
     size_t off = 0;
@@ -63,8 +70,7 @@ Ws carve(void* base, int rows, int V, size_t* total, size_t* zero_bytes) {
         off += align256(bytes);
         return reinterpret_cast<void*>(p);
     };
-    w.gcnt = (unsigned*)take((size_t)rows * 256 * 4);
-    w.gsum = (unsigned long long*)take((size_t)rows * 256 * 8);
+    w.gsum = (unsigned long long*)take((size_t)rows * kBins * 8);
     w.arrived = (unsigned*)take((size_t)rows * 4);
     if (zero_bytes) *zero_bytes = off;
     w.buf = (double*)take((size_t)rows * V * 8);
@@ -73,8 +79,9 @@ Ws carve(void* base, int rows, int V, size_t* total, size_t* zero_bytes) {
     w.pemax = (double*)take((size_t)rows * kBlocks * 8);
     w.psum2 = (double*)take((size_t)rows * kBlocks * 8);
     w.pmass = (double*)take((size_t)rows * kBlocks * 8);
-    w.hcnt = (unsigned*)take((size_t)rows * kBlocks * 256 * 4);
-    w.sel = (unsigned long long*)take((size_t)rows * 8 * 8);
+    w.sel = (unsigned long long*)take((size_t)rows * 2 * 8);
+    w.cand = (unsigned long long*)take((size_t)rows * V * 8);
+    w.ncand = (unsigned*)take((size_t)rows * kBlocks * 4);
     if (total) *total = off;
     return w;
 }
@@ -84,6 +91,7 @@ struct Args {
     int ls, V, mode;
     double T;
     bool topp;
+    unsigned long long target;  // top_p in 2^-60 fixed point, rounded up
     Ws w;
     unsigned long long* rng;
     const int* state;
@@ -224,95 +232,36 @@ __device__ inline double denom(const Args& a, int b) {
     return row_sum((a.mode == AR_SAMPLE_TOKEN ? a.w.psum : a.w.psum2) + b * kBlocks);
 }
 
-// The digit choice of one pass (wavefront 0 of the last chunk): the highest non-empty bucket d
-// with above + sum(buckets >= d) >= target, scanning buckets in descending order, 4 per lane.
-__device__ void select_digit(const Args& a, int b, int level, unsigned long long target, const unsigned* cnt,
-                             const unsigned long long* sm) {
-    const int lane = threadIdx.x & 63;
-    unsigned long long* sel = a.w.sel + b * 8;
-    // state left by the previous pass (nothing before the first)
-    const unsigned long long prefix0 = level ? sel[0] : 0ull;
-    const unsigned long long above = level ? sel[1] : 0ull;
-    unsigned long long lsum = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) lsum += sm[255 - 4 * lane - k];
-    const unsigned long long before = wave_incl_scan(lsum) - lsum;  // buckets above this lane's four
-    unsigned long long acc = above + before;
-    int hit = -1;
-    unsigned long long acc_hit = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int d = 255 - 4 * lane - k;
-        if (hit < 0 && cnt[d] && acc + sm[d] >= target) {
-            hit = d;
-            acc_hit = acc;
-        }
-        acc += sm[d];
-    }
-    const unsigned long long hits = __ballot(hit >= 0);
-    if (!hits) {  // the whole row sums to less than top_p: the reference keeps every value
-        if (lane == 0) sel[2] = 1;
-        return;
-    }
-    if (lane != __builtin_ctzll(hits)) return;
-    const int shift = 56 - 8 * level;
-    const unsigned long long prefix = prefix0 | ((unsigned long long)hit << shift);
-    sel[0] = prefix;  // prefix
-    sel[1] = acc_hit; // fixed-point sum of the values above the prefix range
-    unsigned long long done = 0, take = 0;  // done: 0 searching, 1 keep everything, 2 cut found
-    if (level == 7) {
-        const double pstar = __longlong_as_double((long long)prefix);
-        const unsigned long long pf = (unsigned long long)(pstar * kFix);
-        const unsigned long long ties = cnt[hit];
-        take = 1;
-        if (target > acc_hit) take = pf ? (target - acc_hit + pf - 1) / pf : ties;
-        take = take < 1 ? 1 : (take > ties ? ties : take);
-        done = 2;
-    }
-    sel[2] = done;
-    sel[3] = take;  // values == p* kept
+// Bucket of a probability in [0, 1]: exponent and four mantissa bits, 1.0 in the last one, everything
+// under 2^-63.9 in the first.
+__device__ inline int bucket_of(double p) {
+    const int d = (int)((unsigned long long)__double_as_longlong(p) >> 48) - (0x3FF0 - (kBins - 1));
+    return min(max(d, 0), kBins - 1);
 }
 
-// 4. nucleus search, pass `level`: histogram of digit (key >> shift) & 255 over the keys that match
-//    the prefix chosen so far; the last chunk to arrive picks the digit
-__global__ __launch_bounds__(kThreads) void smp_hist_kernel(Args a, int level, unsigned long long target) {
-    __shared__ unsigned cnt[256];
-    __shared__ unsigned long long sm[256];
+// 4. nucleus search, the whole row: probabilities (written back over the exponentials) into the buckets;
+//    the last chunk to arrive picks the highest bucket d with sum(buckets >= d) >= target
+__global__ __launch_bounds__(kThreads) void smp_bucket_kernel(Args a) {
+    __shared__ unsigned long long sm[kBins], red[kWaves];
     __shared__ int last_s;
+    static_assert(kBins == kThreads, "one bucket per thread");
     const int blk = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
-    if (t < 256) {
-        cnt[t] = 0;
-        sm[t] = 0;
-    }
+    sm[t] = 0;
     __syncthreads();
     int c0, c1;
     chunk_of(a.V, blk, &c0, &c1);
     const double D = denom(a, b);
-    const int shift = 56 - 8 * level;
-    const int hs = level ? shift + 8 : 0;  // bits above the current digit (none at level 0)
-    const unsigned long long want = level ? a.w.sel[b * 8 + 0] >> hs : 0ull;
-    const bool searching = level == 0 || a.w.sel[b * 8 + 2] == 0;
-    const double* buf = a.w.buf + (size_t)b * a.V;
-    if (searching) {
-        for (int i = c0 + t; i < c1; i += kThreads) {
-            const double p = buf[i] / D;
-            const unsigned long long key = (unsigned long long)__double_as_longlong(p);
-            if (level == 0 || (key >> hs) == want) {
-                const int d = (int)((key >> shift) & 255);
-                atomicAdd(&cnt[d], 1u);
-                atomicAdd(&sm[d], (unsigned long long)(p * kFix));
-            }
-        }
+    double* buf = a.w.buf + (size_t)b * a.V;
+    for (int i = c0 + t; i < c1; i += kThreads) {
+        const double p = buf[i] / D;
+        buf[i] = p;
+        const unsigned long long f = (unsigned long long)(p * kFix);
+        if (f) atomicAdd(&sm[bucket_of(p)], f);
     }
     __syncthreads();
-    if (t < 256) {
-        a.w.hcnt[((size_t)b * kBlocks + blk) * 256 + t] = cnt[t];
-        if (cnt[t]) {
-            __hip_atomic_fetch_add(a.w.gcnt + b * 256 + t, cnt[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(a.w.gsum + b * 256 + t, sm[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);  // this thread's histogram atomics have completed
+    unsigned long long* g = a.w.gsum + (size_t)b * kBins + t;
+    if (sm[t]) __hip_atomic_fetch_add(g, sm[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);  // this thread's atomics have completed
     __syncthreads();
     if (t == 0) {
         unsigned* c = a.w.arrived + b;
@@ -323,35 +272,57 @@ __global__ __launch_bounds__(kThreads) void smp_hist_kernel(Args a, int level, u
     }
     __syncthreads();
     if (!last_s) return;
-    // the row histogram, read once and cleared for the next pass
-    if (t < 256) {
-        cnt[t] = __hip_atomic_load(a.w.gcnt + b * 256 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sm[t] = __hip_atomic_load(a.w.gsum + b * 256 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(a.w.gcnt + b * 256 + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(a.w.gsum + b * 256 + t, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // thread t takes bucket kBins - 1 - t: an inclusive scan in thread order sums the buckets from the top
+    g = a.w.gsum + (size_t)b * kBins + (kBins - 1 - t);
+    const unsigned long long mine = __hip_atomic_load(g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long incl = block_incl_scan(mine, red);
+    unsigned long long* sel = a.w.sel + b * 2;
+    // the whole row may sum to less than top_p (the reference then keeps every value): no bucket
+    if (t == kThreads - 1 && (incl < a.target || incl == 0)) sel[0] = ~0ull;
+    const unsigned long long before = incl - mine;
+    if (mine && incl >= a.target && (before < a.target || before == 0)) {
+        sel[0] = (unsigned long long)(kBins - 1 - t);
+        sel[1] = before;
     }
-    __syncthreads();
-    if (t < 64 && searching) select_digit(a, b, level, target, cnt, sm);
 }
 
-// Membership of the nucleus: values > p* and the first `take` (by index) of the values == p*.
-struct Nucleus {
-    int mode;                   // 0: everything (no top-p), 1: everything (top-p kept all), 2: cut
-    unsigned long long pstar, take;
-};
-
-__device__ inline Nucleus nucleus_of(const Args& a, int b) {
-    Nucleus n{0, 0, 0};
-    if (!a.topp) return n;
-    const unsigned long long* sel = a.w.sel + b * 8;
-    if (sel[2] != 2) {
-        n.mode = 1;
-        return n;
+// 5. nucleus search, the bucket of p*: its values' bit patterns in index order, and the mass above it
+__global__ __launch_bounds__(kThreads) void smp_cand_kernel(Args a) {
+    __shared__ double red[kWaves];
+    __shared__ int wcnt[kWaves];
+    const int blk = blockIdx.x, b = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int c0, c1;
+    chunk_of(a.V, blk, &c0, &c1);
+    const unsigned long long sel = a.w.sel[b * 2];
+    const bool cut = sel != ~0ull;
+    const int bin = cut ? (int)sel : -1;  // (no cut: everything lies above)
+    const double* buf = a.w.buf + (size_t)b * a.V;
+    unsigned long long* cand = a.w.cand + (size_t)b * a.V + c0;
+    double s = 0.0;
+    int n = 0;  // values copied so far (the same in every thread)
+    for (int i0 = c0; i0 < c1; i0 += kThreads) {
+        const int i = i0 + t;
+        const double p = i < c1 ? buf[i] : 0.0;
+        const int d = bucket_of(p);
+        if (i < c1 && (!cut || d > bin)) s += p;
+        const bool in = i < c1 && cut && d == bin;
+        const unsigned long long hits = __ballot(in);
+        if (lane == 0) wcnt[wave] = __popcll(hits);
+        __syncthreads();
+        int at = n;
+        for (int w = 0; w < kWaves; w++) {
+            if (w < wave) at += wcnt[w];
+            n += wcnt[w];
+        }
+        if (in) cand[at + __popcll(hits & ((1ull << lane) - 1))] = (unsigned long long)__double_as_longlong(p);
+        __syncthreads();
     }
-    n.mode = 2;
-    n.pstar = sel[0];
-    n.take = sel[3];
-    return n;
+    s = block_sum_d(s, red);
+    if (t == 0) {
+        a.w.pmass[b * kBlocks + blk] = s;
+        a.w.ncand[b * kBlocks + blk] = (unsigned)n;
+    }
 }
 
 __device__ inline void thread_range(int c0, int c1, int* r0, int* r1) {
@@ -360,52 +331,185 @@ __device__ inline void thread_range(int c0, int c1, int* r0, int* r1) {
     *r1 = min(c1, *r0 + per);
 }
 
-// Number of values == p* before this thread's contiguous range: earlier chunks (their last-pass
-// histograms) plus earlier threads of this chunk (a block scan).
-__device__ inline unsigned long long tie_base(const Args& a, const Nucleus& n, int b, int blk, int r0, int r1,
-                                              double D, unsigned long long* red) {
-    unsigned long long mine = 0;
-    if (n.mode == 2) {
-        const double* buf = a.w.buf + (size_t)b * a.V;
-        for (int i = r0; i < r1; i++)
-            mine += (unsigned long long)__double_as_longlong(buf[i] / D) == n.pstar;
-    }
-    unsigned long long before_chunk = 0;
-    if (n.mode == 2) {
-        const int lane = threadIdx.x & 63;
-        const int d = (int)(n.pstar & 255);
-        unsigned long long v = lane < blk ? a.w.hcnt[((size_t)b * kBlocks + lane) * 256 + d] : 0ull;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        before_chunk = v;
-    }
-    return before_chunk + block_incl_scan(mine, red) - mine;
-}
-
-__device__ inline double kept(const Nucleus& n, double q, unsigned long long* rank) {
-    if (n.mode != 2) return q;
-    const unsigned long long key = (unsigned long long)__double_as_longlong(q);
-    if (key > n.pstar) return q;
-    if (key == n.pstar) return (*rank)++ < n.take ? q : 0.0;
-    return 0.0;
-}
-
-// 5. kept probability mass per chunk (before the nucleus renormalisation)
+// 5'. (no nucleus) probability mass per chunk
 __global__ __launch_bounds__(kThreads) void smp_mass_kernel(Args a) {
-    __shared__ unsigned long long ured[kWaves];
     __shared__ double red[kWaves];
     const int blk = blockIdx.x, b = blockIdx.y;
     int c0, c1, r0, r1;
     chunk_of(a.V, blk, &c0, &c1);
     thread_range(c0, c1, &r0, &r1);
     const double D = denom(a, b);
-    const Nucleus n = nucleus_of(a, b);
-    unsigned long long rank = tie_base(a, n, b, blk, r0, r1, D, ured);
     const double* buf = a.w.buf + (size_t)b * a.V;
     double s = 0.0;
-    for (int i = r0; i < r1; i++) s += kept(n, buf[i] / D, &rank);
+    for (int i = r0; i < r1; i++) s += buf[i] / D;
     s = block_sum_d(s, red);
     if (threadIdx.x == 0) a.w.pmass[b * kBlocks + blk] = s;
+}
+
+// The nucleus: values > p*, and the first `take` (by index) of the values == p*.
+struct Nucleus {
+    bool cut;  // false: every value is kept
+    unsigned long long pstar, take;
+};
+
+__device__ inline double kept(const Nucleus& n, double q, unsigned long long* rank) {
+    if (!n.cut) return q;
+    const unsigned long long key = (unsigned long long)__double_as_longlong(q);
+    if (key > n.pstar) return q;
+    if (key == n.pstar) return (*rank)++ < n.take ? q : 0.0;
+    return 0.0;
+}
+
+// LDS of the drawing block's end of the nucleus search
+struct SearchLds {
+    unsigned long long key[kCandLds];  // the bucket's values (when they fit), in index order
+    unsigned long long sum[256];
+    unsigned cnt[256];
+    unsigned off[kBlocks + 1];         // first value of each chunk in that order
+    unsigned long long ties[kBlocks];  // values == p* in the chunks before each chunk
+    double mass[kBlocks];              // kept mass of each chunk
+    unsigned long long prefix, above, pstar, take;
+    unsigned left;
+};
+
+// p*, the ties kept, and the kept mass of every chunk (L.mass), by the whole block.
+__device__ Nucleus finish_search(const Args& a, int b, SearchLds& L) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const unsigned long long bin = a.w.sel[b * 2];
+    if (t < kBlocks) L.mass[t] = a.w.pmass[b * kBlocks + t];
+    if (bin == ~0ull) {
+        __syncthreads();
+        return Nucleus{false, 0, 0};
+    }
+    if (t < kBlocks) {
+        const unsigned c = a.w.ncand[b * kBlocks + t], incl = wave_incl_scan(c);
+        L.off[t + 1] = incl;
+        if (t == 0) L.off[0] = 0;
+    }
+    if (t == 0) {
+        L.prefix = (unsigned long long)(0x3FF0 - (kBins - 1) + (int)bin) << 48;
+        L.above = a.w.sel[b * 2 + 1];
+    }
+    __syncthreads();
+    const unsigned n = L.off[kBlocks];
+    const bool in_lds = n <= (unsigned)kCandLds;
+    // chunk by chunk, a wavefront each: f(chunk, value index, key) for every copied value
+    auto each = [&](auto&& f) {
+        for (int c = wave; c < kBlocks; c += kWaves) {
+            int c0, c1;
+            chunk_of(a.V, c, &c0, &c1);
+            const unsigned long long* src = a.w.cand + (size_t)b * a.V + c0;
+            const unsigned o = L.off[c], m = L.off[c + 1] - o;
+            for (unsigned i0 = 0; i0 < m; i0 += 64) {
+                const unsigned i = i0 + lane;
+                const bool live = i < m;
+                f(c, o + i, live ? (in_lds ? L.key[o + i] : src[i]) : 0ull, live);
+            }
+        }
+    };
+    if (in_lds) {  // 16 lanes a chunk: usually one load each
+        int c0, c1;
+        const int c = t / (kThreads / kBlocks);
+        chunk_of(a.V, c, &c0, &c1);
+        const unsigned o = L.off[c], m = L.off[c + 1] - o;
+        for (unsigned i = t % (kThreads / kBlocks); i < m; i += kThreads / kBlocks)
+            L.key[o + i] = a.w.cand[(size_t)b * a.V + c0 + i];
+    }
+    // radix descent: the highest digit d with above + sum(digits >= d) >= target at each level
+    for (int shift = 40;; shift -= 8) {
+        if (t < 256) {
+            L.cnt[t] = 0;
+            L.sum[t] = 0;
+        }
+        __syncthreads();
+        const unsigned long long want = L.prefix >> (shift + 8), above = L.above;
+        each([&](int, unsigned, unsigned long long key, bool live) {
+            if (live && (key >> (shift + 8)) == want) {
+                const int d = (int)((key >> shift) & 255);
+                atomicAdd(&L.cnt[d], 1u);
+                atomicAdd(&L.sum[d], (unsigned long long)(__longlong_as_double((long long)key) * kFix));
+            }
+        });
+        __syncthreads();
+        if (t < 64) {
+            unsigned long long lsum = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) lsum += L.sum[255 - 4 * lane - k];
+            unsigned long long acc = above + wave_incl_scan(lsum) - lsum;  // the digits above this lane's four
+            int hit = -1;
+            unsigned long long acc_hit = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int d = 255 - 4 * lane - k;
+                if (hit < 0 && L.cnt[d] && acc + L.sum[d] >= a.target) {
+                    hit = d;
+                    acc_hit = acc;
+                }
+                acc += L.sum[d];
+            }
+            const unsigned long long hits = __ballot(hit >= 0);  // (the bucket holds p*: never empty)
+            if (hits && lane == __builtin_ctzll(hits)) {
+                L.prefix |= (unsigned long long)hit << shift;
+                L.above = acc_hit;
+                L.left = L.cnt[hit];
+            }
+        }
+        __syncthreads();
+        if (shift == 0 || L.left == 1) {
+            // every value left has the prefix's bits: one value, or equal ones
+            const unsigned long long pre = L.prefix >> shift;
+            each([&](int, unsigned, unsigned long long key, bool live) {
+                if (live && (key >> shift) == pre) L.pstar = key;
+            });
+            break;
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        const unsigned long long pf = (unsigned long long)(__longlong_as_double((long long)L.pstar) * kFix);
+        unsigned long long take = 1;  // values == p* kept
+        if (a.target > L.above) take = pf ? (a.target - L.above + pf - 1) / pf : L.left;
+        L.take = take < 1 ? 1 : (take > L.left ? L.left : take);
+    }
+    __syncthreads();
+    Nucleus nu{true, L.pstar, L.take};
+    // ties before each chunk, then the kept mass of the bucket's values per chunk (lane sums in index
+    // order, then the lanes): added to the mass above the bucket
+    for (int c = wave; c < kBlocks; c += kWaves)
+        if (lane == 0) L.ties[c] = 0;
+    each([&](int c, unsigned, unsigned long long key, bool live) {
+        const unsigned long long hits = __ballot(live && key == nu.pstar);
+        if (lane == 0) L.ties[c] += __popcll(hits);
+    });
+    __syncthreads();
+    if (t < kBlocks) {
+        const unsigned long long v = L.ties[t], incl = wave_incl_scan(v);
+        L.ties[t] = incl - v;
+    }
+    __syncthreads();
+    double s = 0.0;
+    int cur = -1;
+    unsigned long long rank = 0;
+    auto flush = [&]() {
+        if (cur < 0) return;
+        const double total = wave_sum_d(s);
+        if (lane == 0) L.mass[cur] += total;
+        s = 0.0;
+    };
+    each([&](int c, unsigned, unsigned long long key, bool live) {
+        if (c != cur) {
+            flush();
+            cur = c;
+            rank = L.ties[c];
+        }
+        const unsigned long long hits = __ballot(live && key == nu.pstar);
+        const bool tie = live && key == nu.pstar && rank + __popcll(hits & ((1ull << lane) - 1)) < nu.take;
+        if (live && (key > nu.pstar || tie)) s += __longlong_as_double((long long)key);
+        rank += __popcll(hits);
+    });
+    flush();
+    __syncthreads();
+    return nu;
 }
 
 __device__ inline double java_next_double(unsigned long long* s) {
@@ -419,8 +523,10 @@ __device__ inline double java_next_double(unsigned long long* s) {
     return (double)((hi << 27) + lo) * 0x1.0p-53;
 }
 
-// 6. one block per row: the uniform draw and the index whose cumulative interval holds it
+// 6. one block per row: the end of the nucleus search, the uniform draw and the index whose cumulative
+//    interval holds it
 __global__ __launch_bounds__(kThreads) void smp_draw_kernel(Args a) {
+    __shared__ SearchLds L;
     __shared__ unsigned long long ured[kWaves];
     __shared__ double dred[kWaves];
     __shared__ int ifirst[kWaves], ilast[kWaves];
@@ -430,11 +536,11 @@ __global__ __launch_bounds__(kThreads) void smp_draw_kernel(Args a) {
     // The model draws only when the next step feeds a sampled token (past the prompt), as
     // AutoregressiveModel.next applies its sample function (AutoregressiveModel.java:295-308).
     if (a.state && a.state[2] < a.state[1]) return;
-    const double D = denom(a, b);
-    const Nucleus n = nucleus_of(a, b);
+    const double D = a.topp ? 1.0 : denom(a, b);  // (the nucleus search left probabilities in buf)
+    const Nucleus n = a.topp ? finish_search(a, b, L) : Nucleus{false, 0, 0};
     if (t < 64) {
         // chunk masses in index order; the first chunk whose running total exceeds r
-        const double pm = a.w.pmass[b * kBlocks + lane];
+        const double pm = a.topp ? L.mass[lane] : a.w.pmass[b * kBlocks + lane];
         const double Z = a.topp ? wave_sum_d(pm) : 1.0;
         const double m = a.topp ? pm / Z : pm;
         const double incl = wave_incl_scan(m);
@@ -457,8 +563,12 @@ __global__ __launch_bounds__(kThreads) void smp_draw_kernel(Args a) {
         int c0, c1, r0, r1;
         chunk_of(a.V, blk, &c0, &c1);
         thread_range(c0, c1, &r0, &r1);
-        const unsigned long long rank0 = tie_base(a, n, b, blk, r0, r1, D, ured);
         const double* buf = a.w.buf + (size_t)b * a.V;
+        // values == p* before this thread's contiguous range: earlier chunks, earlier threads
+        unsigned long long ties = 0;
+        if (n.cut)
+            for (int i = r0; i < r1; i++) ties += (unsigned long long)__double_as_longlong(buf[i]) == n.pstar;
+        const unsigned long long rank0 = n.cut ? L.ties[blk] + block_incl_scan(ties, ured) - ties : 0;
         const double Z = sh_Z, r = sh_r, c = sh_c;
         double s = 0.0;
         int last = -1;
@@ -563,15 +673,15 @@ int launch_sample(const SampleLaunch& s, hipStream_t st) {
     }
     if (a.topp) {
         // cumulative >= top_p in 2^-60 fixed point (top_p <= 0 keeps the single largest value)
-        const double tp = s.top_p > 0.0 ? ceil(s.top_p * kFix) : 0.0;
-        const unsigned long long target = (unsigned long long)tp;
-        for (int level = 0; level < 8; level++) {
-            hipLaunchKernelGGL(smp_hist_kernel, grid, block, 0, st, a, level, target);
-            AR_LAUNCH_CHECK();
-        }
+        a.target = (unsigned long long)(s.top_p > 0.0 ? ceil(s.top_p * kFix) : 0.0);
+        hipLaunchKernelGGL(smp_bucket_kernel, grid, block, 0, st, a);
+        AR_LAUNCH_CHECK();
+        hipLaunchKernelGGL(smp_cand_kernel, grid, block, 0, st, a);
+        AR_LAUNCH_CHECK();
+    } else {
+        hipLaunchKernelGGL(smp_mass_kernel, grid, block, 0, st, a);
+        AR_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(smp_mass_kernel, grid, block, 0, st, a);
-    AR_LAUNCH_CHECK();
     hipLaunchKernelGGL(smp_draw_kernel, dim3(s.rows), block, 0, st, a);
     AR_LAUNCH_CHECK();
     return AR_HIP_OK;

@@ -89,6 +89,22 @@ def test_sample_op_nucleus_with_ties(ctx, n, top_p):
     assert near <= 1
 
 
+@pytest.mark.parametrize("n,top_p", [(63, 0.9), (4097, 0.7), (151936, 0.5), (151936, -1.0)])
+def test_sample_op_nucleus_buckets(ctx, n, top_p):
+    """The cut inside a bucket of the first pass that holds a whole row of distinct values (more than the
+    drawing block keeps in LDS at the largest n), a row with one certain value (p = 1, the last bucket),
+    one spread over more octaves than there are buckets, and a vocabulary with empty chunks."""
+    print(f"[sample buckets] n={n} top_p={top_p}", flush=True)
+    rng = np.random.default_rng(n)
+    logits = rng.uniform(0.0, 0.02, (4, n)).astype(np.float32)
+    logits[1] = 0.0
+    logits[1, n // 2] = 100.0
+    logits[2] = np.linspace(-120.0, 0.0, n)
+    logits[3] = rng.permutation(np.linspace(-4.0, 4.0, n))
+    near, _ = _run_op(ctx, logits, hw.SAMPLE_TOKEN, 0.9, top_p, seeds=[7, 8, 9, 10], calls=4)
+    assert near <= 1
+
+
 @pytest.mark.parametrize("mode,temperature", [(hw.SAMPLE_MODEL, 0.0), (hw.SAMPLE_TOKEN, 0.0),
                                               (hw.SAMPLE_TOKEN, -1.0)])
 def test_sample_op_greedy_temperatures_draw_nothing(ctx, mode, temperature):
