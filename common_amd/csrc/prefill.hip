@@ -327,11 +327,14 @@ __global__ __launch_bounds__(256) void fold_rmsnorm_rows_f16_v4_kernel(float* x,
     }
 }
 
-// qk_prep_kernel for the whole-vector QK-norm (the reference's) or no QK-norm, with 16-byte accesses
-// and the row's q / k held in registers: thread i takes rotation pairs (f .. f+3, f+hd/2 .. +3) of
-// query pair-group i (and of key pair-group i), so the norm sums, the rotation and the fp16 / cache
-// stores use the values loaded once.  hd % 8 == 0, heads*hd/8 <= QP*256, kv_heads*hd/8 <= 256.
-template <int QP>
+// qk_prep_kernel with 16-byte accesses and the row's q / k held in registers: thread i takes rotation
+// pairs (f .. f+3, f+hd/2 .. +3) of query pair-group i (and of key pair-group i), so the norm sums, the
+// rotation and the fp16 / cache stores use the values loaded once.  Whole-vector QK-norm (or none): one
+// block sum; per head (PH): the hd/8 consecutive lanes holding a head sum it among themselves.
+// hd/8 a power of two, heads*hd/8 <= QP*256, kv_heads*hd/8 <= 256.  Bound by HBM (the fp32 rows in, the
+// cache rows and fp16 copies out).  Per head, 2,048 rows of the 1.7B shape: 22 -> 14 us; 8,192 rows of the
+// 4B shape: 156 -> 67 us.
+template <int QP, bool PH>
 __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
     __shared__ float2 scratch[4];
     const int tid = threadIdx.x;
@@ -343,6 +346,7 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
     const int nq = p.heads * fd4, nk = p.kv_heads * fd4;
     float4 q1[QP], q2[QP], k1 = make_float4(0.f, 0.f, 0.f, 0.f), k2 = k1;
     float2 ss = make_float2(0.f, 0.f);
+    float sq[QP] = {};  // this pair-group's share of a query head's sum (PH)
     // this thread's first v slice, loaded with q and k so its latency overlaps the norms and rotations
     const float4 v0 = tid < kv_dim / 4 ? reinterpret_cast<const float4*>(v)[tid] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -352,8 +356,9 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
             const int h = idx / fd4, f = (idx - h * fd4) * 4;
             q1[j] = *reinterpret_cast<const float4*>(q + (size_t)h * hd + f);
             q2[j] = *reinterpret_cast<const float4*>(q + (size_t)h * hd + fd + f);
-            ss.x += q1[j].x * q1[j].x + q1[j].y * q1[j].y + q1[j].z * q1[j].z + q1[j].w * q1[j].w +
+            sq[j] = q1[j].x * q1[j].x + q1[j].y * q1[j].y + q1[j].z * q1[j].z + q1[j].w * q1[j].w +
                     q2[j].x * q2[j].x + q2[j].y * q2[j].y + q2[j].z * q2[j].z + q2[j].w * q2[j].w;
+            ss.x += sq[j];
         }
     }
     if (tid < nk) {
@@ -363,11 +368,24 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
         ss.y = k1.x * k1.x + k1.y * k1.y + k1.z * k1.z + k1.w * k1.w + k2.x * k2.x + k2.y * k2.y + k2.z * k2.z +
                k2.w * k2.w;
     }
-    float rq = 1.f, rk = 1.f;
-    if (p.q_norm || p.k_norm) {
-        ss = block_sum2(ss, scratch);
-        rq = 1.0f / sqrtf(ss.x / (float)q_dim + p.eps);
-        rk = 1.0f / sqrtf(ss.y / (float)kv_dim + p.eps);
+    float rq[QP], rk = 1.f;
+    if constexpr (PH) {
+        auto head_factor = [&](float v) {  // (the lanes of a head are all live or all idle)
+            for (int off = fd4 / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            return 1.0f / sqrtf(v / (float)hd + p.eps);
+        };
+#pragma unroll
+        for (int j = 0; j < QP; j++) rq[j] = head_factor(sq[j]);
+        rk = head_factor(ss.y);
+    } else {
+        float r = 1.f;
+        if (p.q_norm || p.k_norm) {
+            ss = block_sum2(ss, scratch);
+            r = 1.0f / sqrtf(ss.x / (float)q_dim + p.eps);
+            rk = 1.0f / sqrtf(ss.y / (float)kv_dim + p.eps);
+        }
+#pragma unroll
+        for (int j = 0; j < QP; j++) rq[j] = r;
     }
     const float4* rope = reinterpret_cast<const float4*>(p.rope_tab + (size_t)pos * fd);  // (c, s) pairs
     // normalise (g * x) * r and rotate four pairs: out1 = x1 c - x2 s, out2 = x2 c + x1 s
@@ -393,7 +411,7 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
         if (idx < nq) {
             const int h = idx / fd4, f = (idx - h * fd4) * 4;
             float o1[4], o2[4];
-            rotate(q1[j], q2[j], p.q_norm, (size_t)h * hd, rq, f, o1, o2);
+            rotate(q1[j], q2[j], p.q_norm, (size_t)h * hd, rq[j], f, o1, o2);
             if (p.q32) {
                 float* qo = p.q32 + (size_t)r * q_dim + (size_t)h * hd;
                 *reinterpret_cast<float4*>(qo + f) = make_float4(o1[0], o1[1], o1[2], o1[3]);
@@ -830,7 +848,7 @@ int launch_qk_prep(const PrefillPrep& a, hipStream_t stream) {
     p.T = a.T; p.p0 = a.p0; p.heads = a.heads; p.kv_heads = a.kv_heads; p.hd = a.hd; p.qb = a.qb;
     p.k16 = a.k16; p.Tp = a.Tp; p.rf = a.range_flag; p.q32 = a.q32;
     const int nq = a.heads * a.hd / 8, nk = a.kv_heads * a.hd / 8;
-    const bool v4 = !a.per_head && a.hd % 8 == 0 && a.qkv_stride % 4 == 0 && nk <= 256 && nq <= 4 * 256 &&
+    const bool v4 = (a.hd == 64 || a.hd == 128) && a.qkv_stride % 4 == 0 && nk <= 256 && nq <= 4 * 256 &&
                     (reinterpret_cast<uintptr_t>(a.qkv) & 15) == 0 &&
                     (!a.q_norm || (reinterpret_cast<uintptr_t>(a.q_norm) & 15) == 0) &&
                     (!a.k_norm || (reinterpret_cast<uintptr_t>(a.k_norm) & 15) == 0) &&
@@ -838,14 +856,21 @@ int launch_qk_prep(const PrefillPrep& a, hipStream_t stream) {
                     (reinterpret_cast<uintptr_t>(a.k16) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.q32) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(a.kcache) & 15) == 0 &&
                     (reinterpret_cast<uintptr_t>(a.vcache) & 15) == 0;
-    if (v4 && nq <= 256)
-        hipLaunchKernelGGL(qk_prep_v4_kernel<1>, dim3(a.B * a.T), dim3(256), 0, stream, p);
-    else if (v4 && nq <= 512)
-        hipLaunchKernelGGL(qk_prep_v4_kernel<2>, dim3(a.B * a.T), dim3(256), 0, stream, p);
-    else if (v4)
-        hipLaunchKernelGGL(qk_prep_v4_kernel<4>, dim3(a.B * a.T), dim3(256), 0, stream, p);
-    else
+#define AR_PREP(QPV)                                                                            \
+    if (a.per_head)                                                                             \
+        hipLaunchKernelGGL((qk_prep_v4_kernel<QPV, true>), dim3(a.B * a.T), dim3(256), 0, stream, p);  \
+    else                                                                                        \
+        hipLaunchKernelGGL((qk_prep_v4_kernel<QPV, false>), dim3(a.B * a.T), dim3(256), 0, stream, p)
+    if (v4 && nq <= 256) {
+        AR_PREP(1);
+    } else if (v4 && nq <= 512) {
+        AR_PREP(2);
+    } else if (v4) {
+        AR_PREP(4);
+    } else {
         hipLaunchKernelGGL(qk_prep_kernel, dim3(a.B * a.T), dim3(256), 0, stream, p);
+    }
+#undef AR_PREP
     AR_LAUNCH_CHECK();
     if (a.q32) return AR_HIP_OK;  // fp32 path: attention reads the fp32 cache rows directly
     AR_CHECK_ARG(a.Tp % 128 == 0 && a.Tp >= a.T, "qk prep: Vᵀ rows %d not a multiple of 128 covering %d", a.Tp, a.T);

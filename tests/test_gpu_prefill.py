@@ -235,7 +235,9 @@ def test_prefill_fp32_weights_vs_oracle(ctx):
 
 
 @pytest.mark.parametrize("heads,kv,hd,T,batch", [(4, 4, 64, 1, 1), (4, 2, 64, 31, 2), (8, 2, 128, 33, 1),
-                                                 (8, 1, 64, 128, 1), (2, 2, 128, 130, 3), (16, 8, 128, 97, 1)])
+                                                 (8, 1, 64, 128, 1), (2, 2, 128, 130, 3), (16, 8, 128, 97, 1),
+                                                 # (row preparation: two and four query pair-groups a thread)
+                                                 (32, 8, 128, 35, 1), (48, 12, 128, 5, 1)])
 def test_prefill_fp32_attention_tiles_vs_oracle(ctx, heads, kv, hd, T, batch):
     """The fp32 prompt attention at the edges of its 32-row tiles and four key slices (fewer tiles than
     slices, one row past a tile, one tile past the slices), every heads-per-KV-head ratio and both
