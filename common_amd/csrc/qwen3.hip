@@ -102,7 +102,7 @@ struct ar_qwen3 {
     void* smp_work = nullptr;
     float2* rope_tab = nullptr;             // [S][hd/2] (cos, sin), computed in double on the host
     int* tokens = nullptr;    // [B][S+1]
-    int* state = nullptr;     // {current position, prompt length, next position}
+    int* state = nullptr;     // {current position, prompt length, next position, step-begin blocks arrived}
     float* staging = nullptr; // fp32 upload staging for dtype conversion
     size_t staging_floats = 0;
     int max_splits = 1;
