@@ -48,6 +48,33 @@ def test_gemm_store_bias(ctx, M, N, K):
     assert rel_err(got, ref) <= 1e-5
 
 
+@pytest.mark.parametrize("M,shift", [(2048, 0), (2043, 0), (2043, 2)])
+def test_gemm_swiglu_paired_stores(ctx, M, shift):
+    """The large-tile SwiGLU epilogue: two columns per store, rows past M (odd M: a pair straddles the
+    end), an output off 4-byte boundaries, and gates far past exp's range on both sides.  One bf16
+    rounding: 2^-8 of the largest value."""
+    N, K = 4096, 64
+    r = np.random.default_rng(M + shift)
+    A = bf16(r.standard_normal((M, K)))
+    W = bf16(r.standard_normal((N, K)) * 0.3)
+    W[::7] = bf16(W[::7] * 100.0)
+    W2 = bf16(r.standard_normal((N, K)) * 0.05)
+    guard = 64
+    Od = ctx.to_device(np.full(M * N + guard, 0x7F7F, np.uint16))
+    view = type("At", (), {"ptr": Od.ptr + shift})()
+    ctx.gemm_bf16(ctx.to_device(bits(A)), ctx.to_device(bits(W)), M, N, K, hw.GEMM_SWIGLU,
+                  W2=ctx.to_device(bits(W2)), O=view)
+    ctx.synchronize()
+    raw = Od.download(np.uint16, M * N + guard)
+    got = (raw[shift // 2:shift // 2 + M * N].astype(np.uint32) << 16).view(np.float32).reshape(M, N)
+    assert (raw[shift // 2 + M * N:] == 0x7F7F).all()
+    g = A.astype(np.float64) @ W.astype(np.float64).T
+    u = A.astype(np.float64) @ W2.astype(np.float64).T
+    with np.errstate(over="ignore"):
+        ref = u * (g / (1 + np.exp(-g)))
+    assert rel_err(got, ref) <= 2.0 ** -8
+
+
 def test_gemm_residual_and_swiglu(ctx):
     M, N, K = 200, 384, 512
     r = np.random.default_rng(9)
