@@ -435,42 +435,47 @@ __global__ __launch_bounds__(NT) void attn_decode_kernel(AttnParams p) {
 }
 
 // Merges the split partials of every query head: o = sum_s e^(m_s - M) o_s / sum_s e^(m_s - M) l_s.
-// Every load that does not depend on the position (the partial outputs of the first kMergeRegs
-// splits and this thread's (m, l) pair) is issued together with the position load, so the merge
-// costs one memory round trip; splits past kMergeRegs (long contexts) are read afterwards.
-template <int HD>
-__global__ __launch_bounds__(HD) void attn_combine_kernel(AttnParams p) {
-    constexpr int kMergeRegs = 32;
+// NG groups of HD threads take every NGth split.  Every load that does not depend on the position (a
+// thread's first kMergeRegs partial outputs and its (m, l) pair) is issued together with the position
+// load, so the merge costs one memory round trip; splits past NG * kMergeRegs are read afterwards.
+// One group covers 32 splits; above that four do (96 splits x 32 heads: 4.8 us, 7.3 with one group, whose
+// loads past the 32nd wait one after another).
+template <int HD, int NG>
+__global__ __launch_bounds__(HD * NG) void attn_combine_kernel(AttnParams p) {
+    constexpr int kMergeRegs = 32, NT = HD * NG;
     __shared__ float w_s[kMaxSplits];
-    __shared__ float red[HD / 64];
-    const int h = blockIdx.x, b = blockIdx.y, i = threadIdx.x;
-    const int lane = i & 63, wave = i >> 6;
+    __shared__ float red[NT / 64];
+    __shared__ float og[NG > 1 ? (NG - 1) * HD : 1];
+    const int h = blockIdx.x, b = blockIdx.y, t = threadIdx.x, i = NG == 1 ? t : t % HD,
+              grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(t / HD);
+    const int lane = t & 63, wave = t >> 6;
     const size_t slot0 = ((size_t)b * p.heads + h) * p.max_splits;
     float ov[kMergeRegs];
 #pragma unroll
-    for (int s = 0; s < kMergeRegs; s++) ov[s] = s < p.max_splits ? p.part_o[(slot0 + s) * HD + i] : 0.f;
-    const float2 ml = i < p.max_splits ? reinterpret_cast<const float2*>(p.part_ml)[slot0 + i]
+    for (int s = 0; s < kMergeRegs; s++)
+        ov[s] = grp + NG * s < p.max_splits ? p.part_o[(slot0 + grp + NG * s) * HD + i] : 0.f;
+    const float2 ml = t < p.max_splits ? reinterpret_cast<const float2*>(p.part_ml)[slot0 + t]
                                        : make_float2(-INFINITY, 0.f);
     const int pos = p.pos ? *p.pos : p.pos_value;
     if (pos < 0 || pos >= p.max_seq) return;
     int nsplit, tile;
     attn_split_plan(pos + 1, p.max_splits, &nsplit, &tile);
     if (nsplit == 1) return;  // the attention kernel wrote the output itself
-    float m_loc = i < nsplit ? ml.x : -INFINITY;
-    for (int s = i + HD; s < nsplit; s += HD) m_loc = fmaxf(m_loc, p.part_ml[(slot0 + s) * 2]);
+    float m_loc = t < nsplit ? ml.x : -INFINITY;
+    for (int s = t + NT; s < nsplit; s += NT) m_loc = fmaxf(m_loc, p.part_ml[(slot0 + s) * 2]);
     m_loc = wave_max_lane63(m_loc);
     if (lane == 63) red[wave] = m_loc;
     __syncthreads();
     float M = red[0];
 #pragma unroll
-    for (int w = 1; w < HD / 64; w++) M = fmaxf(M, red[w]);
+    for (int w = 1; w < NT / 64; w++) M = fmaxf(M, red[w]);
     float l_loc = 0.f;
-    if (i < nsplit) {
+    if (t < nsplit) {
         const float w = expf(ml.x - M);
-        w_s[i] = w;
+        w_s[t] = w;
         l_loc = fmaf(ml.y, w, l_loc);
     }
-    for (int s = i + HD; s < nsplit; s += HD) {
+    for (int s = t + NT; s < nsplit; s += NT) {
         const float w = expf(p.part_ml[(slot0 + s) * 2] - M);
         w_s[s] = w;
         l_loc = fmaf(p.part_ml[(slot0 + s) * 2 + 1], w, l_loc);
@@ -481,12 +486,19 @@ __global__ __launch_bounds__(HD) void attn_combine_kernel(AttnParams p) {
     __syncthreads();
     float L = 0.f;
 #pragma unroll
-    for (int w = 0; w < HD / 64; w++) L += red[w];
+    for (int w = 0; w < NT / 64; w++) L += red[w];
     float O = 0.f;
 #pragma unroll
     for (int s = 0; s < kMergeRegs; s++)
-        if (s < nsplit) O = fmaf(ov[s], w_s[s], O);
-    for (int s = kMergeRegs; s < nsplit; s++) O = fmaf(p.part_o[(slot0 + s) * HD + i], w_s[s], O);
+        if (grp + NG * s < nsplit) O = fmaf(ov[s], w_s[grp + NG * s], O);
+    for (int s = grp + NG * kMergeRegs; s < nsplit; s += NG) O = fmaf(p.part_o[(slot0 + s) * HD + i], w_s[s], O);
+    if constexpr (NG > 1) {
+        if (grp > 0) og[(grp - 1) * HD + i] = O;
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < NG - 1; g++) O += og[g * HD + i];
+    }
     const size_t oi = (size_t)b * p.out_stride + (size_t)h * HD + i;
     p.out[oi] = O / L;
     if (p.out_hi) bf16_planes(O / L, p.out_hi + oi, p.out_lo + oi);
@@ -536,7 +548,10 @@ int launch_t(const AttnLaunch& a, hipStream_t stream) {
         ar_launch((attn_decode_kernel<HD, G, kThreads, KV16, false, 4>), grid, dim3(kThreads), 0, stream, p);
     AR_LAUNCH_CHECK();
     if (a.max_splits > 1) {
-        ar_launch((attn_combine_kernel<HD>), dim3(a.heads, a.batch), dim3(HD), 0, stream, p);
+        if (a.max_splits > 32)
+            ar_launch((attn_combine_kernel<HD, 4>), dim3(a.heads, a.batch), dim3(4 * HD), 0, stream, p);
+        else
+            ar_launch((attn_combine_kernel<HD, 1>), dim3(a.heads, a.batch), dim3(HD), 0, stream, p);
         AR_LAUNCH_CHECK();
     }
     return AR_HIP_OK;
@@ -798,6 +813,17 @@ int attention_max_splits(int max_seq, int kv_heads, int batch, bool kv16) {
     int s = want < cap ? want : cap;
     if (s < need) s = need;
     return s < 1 ? 1 : s;
+}
+
+// The splits of the stand-alone operator for a cache that needs more than one block per CU: whole blocks
+// per CU (32 heads, 8 KV heads, 32,768 rows: 96 splits, three blocks per CU, 55.9 us against 58.5 with the
+// 95 that cover the rows; 16,384 rows: 64, 33.8 against 36.0 with 48).  A model keeps
+// attention_max_splits, measured over its batches (kMaxTile).
+int attention_whole_splits(int max_seq, int kv_heads) {
+    const int s = attention_max_splits(max_seq, kv_heads, 1, false);
+    const int cu = 256 % kv_heads == 0 ? 256 / kv_heads : 1;  // splits of one block per CU
+    const int w = (s + cu - 1) / cu * cu;
+    return s > cu && w <= kMaxSplits ? w : s;
 }
 
 int launch_attention_decode(const AttnLaunch& a, hipStream_t stream) {

@@ -71,7 +71,7 @@ int attention_args(ar_hip_ctx* ctx, const float* q, const float* k, const float*
     a->q = q; a->k = k; a->v = v; a->qkv_stride = 0; a->q_norm = q_norm; a->k_norm = k_norm; a->qk_eps = qk_eps;
     a->per_head_norm = qk_norm_mode == AR_QK_NORM_PER_HEAD; a->kcache = k_cache; a->vcache = v_cache;
     a->max_seq = max_seq; a->pos = nullptr; a->pos_value = pos; a->heads = heads; a->kv_heads = kv_heads;
-    a->head_dim = head_dim; a->rope_theta = rope_theta; a->max_splits = attention_max_splits(max_seq, kv_heads, 1, false);
+    a->head_dim = head_dim; a->rope_theta = rope_theta; a->max_splits = attention_whole_splits(max_seq, kv_heads);
     a->out = out; a->out_stride = heads * head_dim; a->batch = 1;
     return AR_HIP_OK;
 }
@@ -135,9 +135,15 @@ extern "C" int ar_hip_attention_decode_noalloc(ar_hip_ctx* ctx, const float* q, 
     // partial outputs [heads][splits][hd] at the start, (max, sum) pairs [heads][splits][2] after
     // them at a 256-byte boundary.  Nothing needs clearing: the combine uses only the splits this
     // call's attention launch writes (it may load the stale slots past them, never uses them).
-    const size_t o_floats = attention_partial_floats(1, heads, a.max_splits, head_dim);
-    const size_t ml_off = (o_floats + 63) / 64 * 64;
-    const size_t need = ml_off + (size_t)heads * a.max_splits * 2;
+    auto layout = [&](size_t* ml_off) {
+        *ml_off = (attention_partial_floats(1, heads, a.max_splits, head_dim) + 63) / 64 * 64;
+        return *ml_off + (size_t)heads * a.max_splits * 2;
+    };
+    size_t ml_off, need = layout(&ml_off);
+    if (need > kNoAllocScratchFloats) {  // as few splits as cover the cache may still fit
+        a.max_splits = attention_max_splits(max_seq, kv_heads, 1, false);
+        need = layout(&ml_off);
+    }
     AR_CHECK_ARG(need <= kNoAllocScratchFloats,
                  "attention (no-alloc): %d heads x %d splits x (%d + 2) floats of partials exceed the %zu-float "
                  "scratch (cache of %d rows); use ar_hip_attention_decode",
