@@ -15,12 +15,10 @@
 // RMSNorm's 1/sqrt(mean(x^2) + eps) is a per-sequence scalar: the lanes accumulate sum(x^2) from
 // the same loads and the factor scales the finished dot products.
 //
-// A block's wavefronts split the k-steps of a 16-row tile (a gate tile and an up tile for SwiGLU)
-// and sum their 16 x 16 partial tiles through LDS in a fixed order.  Two forms:
-//  * persistent (up to 16 k-steps per wavefront, 12 for SwiGLU: cols <= 4096 / 3072): one
-//    block per CU loops over tiles; each wavefront converts its slice of every input once and keeps
-//    the planes in registers for all tiles; the next tile's weight loads are issued before the
-//    current tile's reduction, so they overlap it;
+// A block's wavefronts split the k-steps of a tile of weight rows and sum their 16 x 16 partial tiles
+// through LDS in a fixed order.  Two forms:
+//  * packed (up to 8 sequences, up to 16 k-steps per wavefront: cols <= 4096): one block per CU loops over
+//    tiles with the input planes in registers (see gemv_mfma_pack_kernel);
 //  * streaming (wider inputs, or fewer tiles than CUs): one tile per 16-wavefront block; each
 //    chunk of k-steps issues its weight and input loads together, and the next chunk's loads are in
 //    flight while the current chunk is converted and multiplied.
@@ -34,16 +32,14 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kPersistWaves = 8;
+constexpr int kPackWaves = 8;
+constexpr int kPackSteps = 16;   // k-steps of a wavefront whose planes stay in registers
 constexpr int kStreamWaves = 16;
 constexpr int kStreamChunk = 2;  // k-steps per load chunk (two chunks in flight)
 constexpr int kMaxKSplit = 4;    // k-slices per tile in the split streaming form
 
-__device__ inline unsigned bf16_bits(float f) {  // round to nearest even; NaN stays NaN
-    unsigned u = __float_as_uint(f);
-    if ((u & 0x7F800000u) == 0x7F800000u) return (u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return u >> 16;
+__device__ inline unsigned bf16_bits(float f) {  // round to nearest even (v_cvt_pk_bf16_f32); NaN stays NaN
+    return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
 // 8 consecutive inputs of one sequence: gain applied when gp is given (sum of squares of the raw
@@ -162,94 +158,217 @@ struct Finish {
     }
 };
 
-// KS: k-steps per wavefront whose planes stay in registers (>= kpw)
+// Up to 8 sequences: one MFMA per k-step carries both planes, lanes 0-7 of each 16-lane row the hi plane of
+// sequences 0-7 and lanes 8-15 the lo plane, so columns b and b + 8 of the result add up to sequence b's
+// products (half the MFMAs and half the plane registers of one MFMA per plane).  A tile is 16 weight
+// rows; for SwiGLU 8 gate rows and the same 8 up rows.
+// One block of 8 wavefronts per CU walks tiles t, t + grid, ...; a wavefront's k-steps of the next SETS
+// tiles are always in flight (register sets, two to four: some 100 KB per CU), across the tile's one barrier, which waits for LDS only
+// (a barrier that waits for the loads too leaves the CU without any request once per tile).  Four
+// wavefronts finish a tile while the others go on.
+// 9,728 x 2,560 SwiGLU, 8 sequences: 26 us a call, 34 with one MFMA per plane, whole 16 + 16-row tiles (608
+// on 256 CUs: 2.4 rounds) and a full barrier; in a decode step of the 4B shape, weights cold in HBM: QKV
+// (6,144 x 2,560) 15.7 -> 13.7 us, 16,896-row head 31 -> 24.  Bound by HBM and, with few tiles per CU, by
+// the first loads' latency and the last round.  8-row tiles for the other epilogues too (QKV in one and a
+// half rounds instead of two) measured slower: 14.7 us, twice the barriers for the same bytes.
 template <int EPI, int KS>
-__global__ __launch_bounds__(kPersistWaves * 64) void gemv_mfma_persist_kernel(gemv::Params p, int kpw, int tiles) {
-    constexpr int NW = kPersistWaves, NMAT = (EPI == GEMV_EPI_SWIGLU) ? 2 : 1;
-    using F = Finish<NW, NMAT, EPI>;
-    __shared__ float cpart[NW][NMAT][256];
-    __shared__ float ssw[NW][16];
-    __shared__ float tot[256];
+__global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv::Params p, int tiles) {
+    constexpr int NW = kPackWaves, SETS = KS <= 6 ? 4 : KS <= 10 ? 3 : 2;  // tiles in flight
+    constexpr bool SW = EPI == GEMV_EPI_SWIGLU;
+    constexpr int TR = SW ? 8 : 16;  // output rows of a tile
+    __shared__ float cpart[2][NW][256];
+    __shared__ float ssw[NW][8];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15,
+              q = lane >> 4, seq = r & 7;
+    const int nsteps = p.cols / 32, s0 = nsteps * w / NW, ns = nsteps * (w + 1) / NW - s0;  // KS - 2 <= ns <= KS
+    const bool live = seq < p.batch, norm = p.norm_w != nullptr;
+    const int step = gridDim.x;
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, q = lane >> 4;
-    const int nsteps = p.cols / 32;
-    const int s0 = w * kpw, ns = max(0, min(kpw, nsteps - s0));  // this wavefront's k-steps
-    const bool live = r < p.batch;
-    const bool norm = p.norm_w != nullptr;
-
-    const uint16_t* wbase[NMAT];
-    wbase[0] = reinterpret_cast<const uint16_t*>(p.w) + (size_t)s0 * 32 + 8 * q;
-    if (NMAT == 2) wbase[NMAT - 1] = reinterpret_cast<const uint16_t*>(p.w2) + (size_t)s0 * 32 + 8 * q;
-    u32x4 wv[NMAT][KS];
-#define AR_MFMA_LOAD_TILE(t_)                                                                         \
-    do {                                                                                              \
-        const size_t ro = (size_t)min((t_) * 16 + r, p.rows - 1) * p.cols;                            \
-        _Pragma("unroll") for (int i = 0; i < KS; i++) if (i < ns) _Pragma("unroll") for (int m = 0; \
-                                                                                         m < NMAT;   \
-                                                                                         m++)        \
-            wv[m][i] = *reinterpret_cast<const u32x4*>(wbase[m] + ro + i * 32);                       \
-    } while (0)
+    // weight rows of this lane in tile t: row t * TR + lane's row of its matrix; tiles past the end read
+    // one line over and over instead of branching, so the waits count loads exactly
+    const uint16_t* const wm = reinterpret_cast<const uint16_t*>(SW && r >= 8 ? p.w2 : p.w);
+    const int lrow = TR == 8 ? r & 7 : r;
+    const size_t koff = (size_t)s0 * 32 + 8 * q;
+    // (a line of its own for every wavefront: one line for all of them is one L2 channel's queue)
+    const uint16_t* const idle = reinterpret_cast<const uint16_t*>(p.w) + (size_t)blockIdx.x * TR * p.cols + s0 * 32;
+    u32x4 wv[SETS][KS];
+    auto load = [&](int set, int t) __attribute__((always_inline)) {
+        const bool in = t < tiles;
+        const uint16_t* src = in ? wm + (size_t)min(t * TR + lrow, p.rows - 1) * p.cols + koff : idle;
+        const int inc = in ? 32 : 0;
+#pragma unroll
+        for (int i = 0; i < KS; i++)  // (steps past ns repeat the last one; never multiplied)
+            wv[set][i] = *reinterpret_cast<const u32x4*>(src + (i < KS - 2 ? i : min(i, ns - 1)) * inc);
+    };
     int t = blockIdx.x;
-    if (t < tiles) AR_MFMA_LOAD_TILE(t);  // weights do not depend on x: their latency overlaps the planes
-    // input planes of this wavefront's k-steps, once for all tiles: read as written by the kernel
-    // that produced the input (the RMSNorm sum of squares still comes from the fp32 input), or
-    // converted here
-    u32x4 hv[KS], lv[KS];
-    float ss = 0.f;
-    {
-        const float* xp = p.x + (size_t)min(r, p.batch - 1) * p.x_stride + (size_t)s0 * 32 + 8 * q;
-        if (p.x_hi) {
-            const size_t po = (size_t)min(r, p.batch - 1) * p.x_stride + (size_t)s0 * 32 + 8 * q;
-            const u32x4 zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int i = 0; i < KS; i++)
-                if (i < ns) {
-                    hv[i] = live ? *reinterpret_cast<const u32x4*>(p.x_hi + po + i * 32) : zero;
-                    lv[i] = live ? *reinterpret_cast<const u32x4*>(p.x_lo + po + i * 32) : zero;
-                }
-            if (norm) {
-#pragma unroll
-                for (int i = 0; i < KS; i++)
-                    if (i < ns) sumsq8(load4(xp + i * 32, live), load4(xp + i * 32 + 4, live), ss);
-            }
-        } else {
-            const float* gp = norm ? p.norm_w + (size_t)s0 * 32 + 8 * q : nullptr;
-#pragma unroll
-            for (int i = 0; i < KS; i++)
-                if (i < ns)
-                    make_planes(load4(xp + i * 32, live), load4(xp + i * 32 + 4, live), gp ? gp + i * 32 : nullptr,
-                                ss, hv[i], lv[i]);
-        }
-    }
-    if (norm) {
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
-        if (q == 0) ssw[w][r] = ss;
-    }
 
-    for (; t < tiles; t += gridDim.x) {
-        floatx4 acc[NMAT];
+    // this lane's plane of its sequence, once for all tiles: as written by the kernel that produced the
+    // input, or converted here.  With planes the RMSNorm sum of squares still comes from the fp32 input:
+    // lane l sums sequence l / 8, and its loads and the planes' go ahead of the weights of two tiles, so
+    // nothing waits behind those and HBM has requests from the start
+    u32x4 pv[KS];
+    float ss = 0.f;
+    const bool planes = p.x_hi != nullptr;
+    const size_t xo = (size_t)min(seq, p.batch - 1) * p.x_stride + koff;
+    if (planes) {
+        float4 xs[KS];
+        const int sseq = lane >> 3;
+        const float* const xrow = p.x + (size_t)min(sseq, p.batch - 1) * p.x_stride + (size_t)s0 * 32 + 4 * (lane & 7);
+        if (norm)
 #pragma unroll
-        for (int m = 0; m < NMAT; m++) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < KS; i++)
+                xs[i] = *reinterpret_cast<const float4*>(xrow + (i < KS - 2 ? i : min(i, ns - 1)) * 32);
+        const uint16_t* const pl = (r < 8 ? p.x_hi : p.x_lo) + xo;
 #pragma unroll
         for (int i = 0; i < KS; i++)
-            if (i < ns)
-#pragma unroll
-                for (int m = 0; m < NMAT; m++) acc[m] = mac2(wv[m][i], hv[i], lv[i], acc[m]);
-        if (t + (int)gridDim.x < tiles) AR_MFMA_LOAD_TILE(t + (int)gridDim.x);  // in flight during the reduction
-#pragma unroll
-        for (int m = 0; m < NMAT; m++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) cpart[w][m][(4 * q + j) * 16 + r] = acc[m][j];
-        __syncthreads();
-        F::outputs(p, cpart, ssw, norm, t * 16, tid, tot);
-        if (EPI == GEMV_EPI_ARGMAX) {
-            __syncthreads();
-            F::argmax(p, tot, t * 16, t, tid);
+            pv[i] = *reinterpret_cast<const u32x4*>(pl + (i < KS - 2 ? i : min(i, ns - 1)) * 32);
+        if (KS <= 12) {  // (registers: above 12 steps after the sums)
+            load(0, t);
+            load(1, t + step);
         }
-        __syncthreads();  // cpart / tot are rewritten by the next tile
+        if (norm) {
+#pragma unroll
+            for (int i = 0; i < KS; i++)
+                if (i < KS - 2 || i < ns) {
+                    ss = fmaf(xs[i].x, xs[i].x, ss);
+                    ss = fmaf(xs[i].y, xs[i].y, ss);
+                    ss = fmaf(xs[i].z, xs[i].z, ss);
+                    ss = fmaf(xs[i].w, xs[i].w, ss);
+                }
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            if ((lane & 7) == 0) ssw[w][sseq] = ss;
+        }
+        if (KS > 12) {
+            load(0, t);
+            load(1, t + step);
+        }
+        if (!live)
+#pragma unroll
+            for (int i = 0; i < KS; i++) pv[i] = u32x4{0u, 0u, 0u, 0u};
+    } else {
+        load(0, t);
+        if (KS <= 12) load(1, t + step);
+#pragma unroll
+        for (int i = 0; i < KS; i++) {
+            const int k = (i < KS - 2 ? i : min(i, ns - 1)) * 32;
+            const bool use = live && (i < KS - 2 || i < ns);
+            u32x4 hi, lo;
+            make_planes(load4(p.x + xo + k, use), load4(p.x + xo + k + 4, use), norm ? p.norm_w + koff + k : nullptr, ss,
+                        hi, lo);
+            pv[i] = r < 8 ? hi : lo;
+        }
+        if (norm) {
+            ss += __shfl_xor(ss, 16, 64);
+            ss += __shfl_xor(ss, 32, 64);
+            if (q == 0 && r < 8) ssw[w][r] = ss;
+        }
+        if (KS > 12) load(1, t + step);
     }
-#undef AR_MFMA_LOAD_TILE
+#pragma unroll
+    for (int k = 2; k < SETS; k++) load(k, t + k * step);
+
+    float rn = 1.f;          // finishing wavefronts: RMSNorm factor of sequence `seq`
+    bool have_rn = false;
+    int par = 0;             // partial-tile buffer of the next tile
+    float best = -INFINITY;  // ARGMAX: this lane's best value and its row over every tile
+    int besti = 0x7FFFFFFF;
+    // rows of a finished tile by lane, gate row and up row of one output 32 lanes apart
+    const int frow = (q & 1) + 2 * w + (q >> 1) * 8;
+    auto tile = [&](int set) __attribute__((always_inline)) {
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < KS; i++)
+            if (i < KS - 2 || i < ns)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[set][i]),
+                                                              __builtin_bit_cast(bf16x8, pv[i]), acc, 0, 0, 0);
+        load(set, t + SETS * step);
+#pragma unroll
+        for (int j = 0; j < 4; j++) cpart[par][w][(4 * q + j) * 16 + r] = acc[j];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the weight loads stay in flight
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        par ^= 1;
+        if (w >= 4) return;
+        if (norm && !have_rn) {
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < NW; k++) s += ssw[k][seq];
+            rn = 1.0f / sqrtf(s / (float)p.cols + p.eps);
+            have_rn = true;
+        }
+        float v = 0.f;
+#pragma unroll
+        for (int k = 0; k < NW; k++) v += cpart[par ^ 1][k][frow * 16 + r];
+        v = (v + __shfl_xor(v, 8, 64)) * rn;  // hi + lo
+        const float up = SW ? __shfl_xor(v, 32, 64) : 0.f;
+        const int row = t * TR + frow;
+        if (r >= 8 || !live || frow >= TR || row >= p.rows) return;
+        if constexpr (EPI == GEMV_EPI_ARGMAX) {
+            if (p.y) p.y[(size_t)seq * p.y_stride + row] = v;
+            if (gemv::better(v, row, best, besti)) {
+                best = v;
+                besti = row;
+            }
+        } else {
+            const size_t o = (size_t)seq * p.y_stride + row;
+            float val;
+            if constexpr (EPI == GEMV_EPI_STORE) {
+                val = p.bias ? v + p.bias[row] : v;
+            } else if constexpr (EPI == GEMV_EPI_RESIDUAL) {
+                val = p.y[o] + v;
+            } else {  // SwiGLU: u * (g * 1/(exp(-g)+1))
+                const float sg = 1.0f / (expf(-v) + 1.0f);
+                val = up * (v * sg);
+            }
+            p.y[o] = val;
+            if (p.y_hi) bf16_planes(p.y_gain ? val * p.y_gain[row] : val, p.y_hi + o, p.y_lo + o);
+        }
+    };
+    while (t < tiles) {
+#pragma unroll
+        for (int k = 0; k < SETS; k++) {
+            tile(k);
+            t += step;
+            if (t >= tiles) break;
+        }
+    }
+    if constexpr (EPI == GEMV_EPI_ARGMAX) {
+        if (w >= 4) return;
+        // the best of this wavefront's rows, then one key per sequence
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float ov = __shfl_xor(best, off, 64);
+            const int oi = __shfl_xor(besti, off, 64);
+            if (gemv::better(ov, oi, best, besti)) {
+                best = ov;
+                besti = oi;
+            }
+        }
+        if (q == 0 && r < 8 && live && besti != 0x7FFFFFFF)
+            atomicMax(p.keys + (size_t)seq * kArgmaxSlots + ((blockIdx.x * 4 + w) & (kArgmaxSlots - 1)),
+                      gemv::argmax_key(best, besti));
+    }
+}
+
+template <int EPI>
+void launch_pack(const gemv::Params& p, int cus, hipStream_t st) {
+    const int rows = EPI == GEMV_EPI_SWIGLU ? 8 : 16, tiles = (p.rows + rows - 1) / rows;
+    const dim3 grid(std::min(tiles, cus)), block(64 * kPackWaves);
+    const int ks = (p.cols / 32 + kPackWaves - 1) / kPackWaves;
+#define AR_PACK(K) \
+    if (ks <= K) return ar_launch((gemv_mfma_pack_kernel<EPI, K>), grid, block, 0, st, p, tiles)
+    AR_PACK(3);
+    AR_PACK(4);
+    AR_PACK(5);
+    AR_PACK(6);
+    AR_PACK(8);
+    AR_PACK(10);
+    AR_PACK(12);
+    AR_PACK(14);
+    AR_PACK(16);
+#undef AR_PACK
 }
 
 // NWS wavefronts per block; ks blocks per 16-row tile (block = tile * ks + k-slice), each taking
@@ -384,24 +503,13 @@ template <int EPI>
 int launch_epi(const gemv::Params& p, hipStream_t st) {
     constexpr int NMAT = (EPI == GEMV_EPI_SWIGLU) ? 2 : 1;
     const int nsteps = p.cols / 32, tiles = (p.rows + 15) / 16;
-    const int kpw_p = (nsteps + kPersistWaves - 1) / kPersistWaves;
-    const int persist = ar_device_cus(st);  // one persistent block per CU of the stream's device
-    // register budget of the persistent form: planes 8*KS + weights 4*NMAT*KS
-    const int ks_max = NMAT == 2 ? 12 : 16;
+    const int persist = ar_device_cus(st);  // one packed block per CU of the stream's device
     // fewer tiles than CUs (the 2560-row projections at C5): one tile per 16-wavefront block spreads
-    // the loads over more wavefronts (measured: O 4096 -> 2560 15.5 us streaming vs 23.7 persistent;
-    // QKV 2560 -> 6144 20.3 us persistent vs 25.6 streaming)
-    if (kpw_p <= ks_max && tiles >= persist) {
-        const dim3 grid(std::min(tiles, persist)), block(64 * kPersistWaves);
-        if (kpw_p <= 4)
-            ar_launch((gemv_mfma_persist_kernel<EPI, 4>), grid, block, 0, st, p, kpw_p, tiles);
-        else if (kpw_p <= 8)
-            ar_launch((gemv_mfma_persist_kernel<EPI, 8>), grid, block, 0, st, p, kpw_p, tiles);
-        else if (kpw_p <= 12)
-            ar_launch((gemv_mfma_persist_kernel<EPI, 12>), grid, block, 0, st, p, kpw_p, tiles);
-        else
-            ar_launch((gemv_mfma_persist_kernel<EPI, (NMAT == 2 ? 12 : 16)>), grid, block, 0, st, p, kpw_p,
-                               tiles);
+    // the loads over more wavefronts (measured: O 4096 -> 2560 15.5 us streaming vs 23.7 with one block per
+    // tile of 8 wavefronts).  The packed form takes up to 16 k-steps per wavefront.
+    if (p.batch <= 8 && nsteps >= kPackWaves && nsteps <= kPackWaves * kPackSteps &&
+        (NMAT == 2 ? (p.rows + 7) / 8 : tiles) >= persist) {
+        launch_pack<EPI>(p, persist, st);
     } else {
         // fewer tiles than CUs and nothing that needs the whole row in one block: split k over
         // ks = 2*CUs / tiles blocks of 8 wavefronts (two per CU), partials folded in order

@@ -34,6 +34,13 @@ def _rng(seed):
     (8200, 2560, 8, True, False, True),
     (20000, 1024, 1, True, False, False),
     (20000, 1024, 6, True, False, True),
+    # packed bf16 form (3-8 sequences): one k-step a wavefront, uneven k-steps, the widest input, tiles one
+    # past whole rounds and a ragged last tile
+    (4096, 256, 8, True, True, True),
+    (4099, 288, 5, True, False, True),
+    (8193, 1184, 3, False, True, True),
+    (4100, 3552, 7, True, False, True),
+    (12289, 4096, 4, True, True, True),
 ])
 def test_dense(ctx, rows, cols, batch, norm, bias, bf16):
     r = _rng(rows * 7 + cols)
@@ -61,7 +68,9 @@ def test_dense(ctx, rows, cols, batch, norm, bias, bf16):
 
 @pytest.mark.parametrize("rows,cols,batch,bf16", [(768, 256, 1, False), (3072, 1024, 1, False),
                                                   (6144, 2048, 2, True), (9728, 2560, 8, True),
-                                                  (3000, 1024, 4, False)])
+                                                  (3000, 1024, 4, False), (2048, 256, 3, True),
+                                                  (2051, 416, 7, True), (4104, 3616, 5, True),
+                                                  (2049, 4096, 8, True)])
 def test_swiglu(ctx, rows, cols, batch, bf16):
     r = _rng(rows + cols)
     Wg = (r.standard_normal((rows, cols)) * 0.02).astype(np.float32)
