@@ -160,7 +160,8 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kernel(Params p, int mt, int 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // (past the last tile the copies re-read it into a stage nobody reads)
+    // (past the last tile the copies re-read it into a stage nobody reads: a branch round them and waits counted
+    // for the tail measured slower, 75.3 -> 76.4 us at 1,021 x 4,096 x 1,024 and 21.3 -> 24.3 at 253 x 704 x 2,080)
 #pragma unroll
     for (int i = 0; i < ST; i++) copy(min(i, nit - 1), i);
     asm volatile("" ::: "memory");
