@@ -330,8 +330,9 @@ __global__ __launch_bounds__(256) void fold_rmsnorm_rows_f16_v4_kernel(float* x,
 // qk_prep_kernel with 16-byte accesses and the row's q / k held in registers: thread i takes rotation
 // pairs (f .. f+3, f+hd/2 .. +3) of query pair-group i (and of key pair-group i), so the norm sums, the
 // rotation and the fp16 / cache stores use the values loaded once.  Whole-vector QK-norm (or none): one
-// block sum; per head (PH): the hd/8 consecutive lanes holding a head sum it among themselves.
-// hd/8 a power of two, heads*hd/8 <= QP*256, kv_heads*hd/8 <= 256.  Bound by HBM (the fp32 rows in, the
+// block sum; per head (PH): the hd/8 consecutive lanes holding a head sum it among themselves, with
+// qk_prep_kernel's roundings, so a head's factor has the same bits in both kernels (the fp16 copies round
+// on it).  hd 64 or 128, heads*hd/8 <= QP*256, kv_heads*hd/8 <= 256.  Bound by HBM (the fp32 rows in, the
 // cache rows and fp16 copies out).  Per head, 2,048 rows of the 1.7B shape: 22 -> 14 us; 8,192 rows of the
 // 4B shape: 156 -> 67 us.
 template <int QP, bool PH>
@@ -346,19 +347,18 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
     const int nq = p.heads * fd4, nk = p.kv_heads * fd4;
     float4 q1[QP], q2[QP], k1 = make_float4(0.f, 0.f, 0.f, 0.f), k2 = k1;
     float2 ss = make_float2(0.f, 0.f);
-    float sq[QP] = {};  // this pair-group's share of a query head's sum (PH)
     // this thread's first v slice, loaded with q and k so its latency overlaps the norms and rotations
     const float4 v0 = tid < kv_dim / 4 ? reinterpret_cast<const float4*>(v)[tid] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < QP; j++) {
         const int idx = tid + 256 * j;
+        q1[j] = q2[j] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (idx < nq) {
             const int h = idx / fd4, f = (idx - h * fd4) * 4;
             q1[j] = *reinterpret_cast<const float4*>(q + (size_t)h * hd + f);
             q2[j] = *reinterpret_cast<const float4*>(q + (size_t)h * hd + fd + f);
-            sq[j] = q1[j].x * q1[j].x + q1[j].y * q1[j].y + q1[j].z * q1[j].z + q1[j].w * q1[j].w +
+            ss.x += q1[j].x * q1[j].x + q1[j].y * q1[j].y + q1[j].z * q1[j].z + q1[j].w * q1[j].w +
                     q2[j].x * q2[j].x + q2[j].y * q2[j].y + q2[j].z * q2[j].z + q2[j].w * q2[j].w;
-            ss.x += sq[j];
         }
     }
     if (tid < nk) {
@@ -370,13 +370,32 @@ __global__ __launch_bounds__(256) void qk_prep_v4_kernel(PrepParams p) {
     }
     float rq[QP], rk = 1.f;
     if constexpr (PH) {
-        auto head_factor = [&](float v) {  // (the lanes of a head are all live or all idle)
-            for (int off = fd4 / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        // qk_prep_kernel sums a head over 64 lanes: hd 128 lane f adds its pair (f, f + 64) with one FMA, hd 64
+        // lanes f and f + 32 add their rounded squares; then lanes f ^ 32 (or 16), ... f ^ 1.  Here a lane
+        // holds f = 4 * (lane % fd4) + e, so the steps down to f ^ 4 cross lanes and f ^ 2, f ^ 1 are the four
+        // sums e: after the first two steps lane bits fd4/2 and fd4/4 name the one e a lane goes on with.
+        // (The lanes of a head are all live or all idle.)
+        const bool b1 = tid & (fd4 / 2), b0 = tid & (fd4 / 4);
+        auto head_factor = [&](float4 a, float4 c) {
+#pragma clang fp contract(off)
+            const float x1[4] = {a.x, a.y, a.z, a.w}, x2[4] = {c.x, c.y, c.z, c.w};
+            float t[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float s1 = x1[e] * x1[e];
+                t[e] = hd == 128 ? __builtin_fmaf(x2[e], x2[e], s1) : s1 + x2[e] * x2[e];
+            }
+            const float k0 = (b1 ? t[2] : t[0]) + __shfl_xor(b1 ? t[0] : t[2], fd4 / 2, 64);
+            const float k1 = (b1 ? t[3] : t[1]) + __shfl_xor(b1 ? t[1] : t[3], fd4 / 2, 64);
+            float v = (b0 ? k1 : k0) + __shfl_xor(b0 ? k0 : k1, fd4 / 4, 64);
+            for (int off = fd4 / 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            v += __shfl_xor(v, fd4 / 2, 64);
+            v += __shfl_xor(v, fd4 / 4, 64);
             return 1.0f / sqrtf(v / (float)hd + p.eps);
         };
 #pragma unroll
-        for (int j = 0; j < QP; j++) rq[j] = head_factor(sq[j]);
-        rk = head_factor(ss.y);
+        for (int j = 0; j < QP; j++) rq[j] = head_factor(q1[j], q2[j]);
+        rk = head_factor(k1, k2);
     } else {
         float r = 1.f;
         if (p.q_norm || p.k_norm) {

@@ -285,6 +285,45 @@ def test_prefill_fp32_attention_tiles_vs_oracle(ctx, heads, kv, hd, T, batch):
         assert rel_err(lp[b], rl[T - 1]) <= 1e-5, rel_err(lp[b], rl[T - 1])
 
 
+def _one_product_weights(cfg, seed):
+    """Weights under which every product of a prompt pass has one non-zero term, so its order does not
+    matter: token t is a multiple of unit vector t, the output projection copies the attention output of the
+    first dim / head_size heads, the FFN adds nothing."""
+    r = np.random.default_rng(seed)
+    sd = synthetic.state_dict(cfg, seed=seed)
+    d, p = cfg.dim, "model.layers.0."
+    out = {k: np.array(v) for k, v in sd.items()}
+    out["model.embed_tokens.weight"] = np.diag(r.uniform(0.5, 2.0, cfg.vocab_size)).astype(np.float32)[:, :d]
+    for n, heads in (("q", cfg.head_count), ("k", cfg.kv_head_count), ("v", cfg.kv_head_count)):
+        w = np.random.default_rng(seed + ord(n)).standard_normal((64 * 128, d)).astype(np.float32)
+        out[p + "self_attn.%s_proj.weight" % n] = np.ascontiguousarray(w[:heads * cfg.head_size])
+        if n != "v":
+            g = np.random.default_rng(seed + 2 * ord(n)).normal(1.0, 0.1, (64, cfg.head_size)).astype(np.float32)
+            out[p + "self_attn.%s_norm.weight" % n] = np.ascontiguousarray(g[:heads])
+    out[p + "self_attn.o_proj.weight"] = np.eye(d, cfg.q_dim, dtype=np.float32)
+    out[p + "mlp.down_proj.weight"] = np.zeros((d, cfg.hidden_dim), np.float32)
+    return out
+
+
+def test_row_preparation_forms_give_the_same_bits(ctx):
+    """Per-head QK-norm of prompt rows: 18 KV heads run the scalar row preparation, 2 the 16-byte form.  The
+    same two heads come out with the same bits: the norm factors are the same fp32 sums, and everything after
+    them sees one head at a time."""
+    hidden = []
+    for heads in (2, 18):
+        cfg = C.Qwen3Config(dim=256, hidden_dim=64, layer_count=1, head_count=heads, kv_head_count=heads,
+                            vocab_size=256, seq_len=48, head_size=128, qk_norm_mode=C.QK_NORM_PER_HEAD)
+        with Qwen3(cfg, _one_product_weights(cfg, seed=11), ctx) as m:
+            for T in (2, 7, 40):
+                m.model.reset()
+                m.model.set_prompt(synthetic.prompt_ids(T, cfg.vocab_size, seed=T))
+                m.model.prefill()
+                hidden.append(m.model.hidden())
+            assert m.model.prefill_by_steps() == 0
+    for a, b in zip(hidden[:3], hidden[3:]):
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_prefill_fp32_c3_prompt_vs_oracle(ctx):
     """BASELINE config 3 (Qwen3-0.6B shape, fp32, q_dim 2048 != dim): the 128-token prompt through
     the fp32 batched prefill, then 8 greedy steps, against the FP32 oracle's batched prompt pass
