@@ -589,11 +589,15 @@ int pick_g(const AttnLaunch& a, hipStream_t s) {
 //   O^T (hd x 32 queries)     += V^T . P^T contraction step r: key (r/4)*8 + (l/32)*4 + r%4 (the
 //                                          result layout of S^T); output row i of tile j is dim
 //                                          NT*i + j, so one load per key row feeds every tile
-// K of the wavefront's next tile is loaded while P.V runs, V while the next Q.K runs.
-// 0.6B shape (16 heads, 8 KV heads, hd 128), 1,531 rows: 100 us (96 TFLOP/s of the causal half; the
-// matrix units are busy 60% of it, the rest is the uneven end of the causal blocks and each block's
-// start and merge) against 382 us for one block per (row, KV head) on the vector units, where each
-// row reads its whole context; 128 rows 10.9 against 11.4 us.
+// K and V of the wavefront's next tile are loaded half a tile at a time, as the registers of the one in use
+// come free.  A score is added up in chains of 16 dims and an output in chains of 8 keys, each chain in one
+// of two accumulators of its own and added to the sum by the vector units while the next one runs: one
+// accumulator for a whole sum (128 dims, a quarter of the keys) was 1.5 to 1.9 times as far from 64 bits as
+// this and as the vector form (3.1e-7, 1.9e-7 and 1.8e-7 at 100 rows), for 98 instead of 109 us.
+// 0.6B shape (16 heads, 8 KV heads, hd 128), 1,531 rows: 109 us (88 TFLOP/s of the causal half, 58% of the
+// matrix rate; the rest is the uneven end of the causal blocks and each block's start and merge) against
+// 382 us for one block per (row, KV head) on the vector units, where each row reads its whole context; 128
+// rows 11.1 against 11.4 us.
 struct PrefillAttnF32 {
     const float *q32, *kcache, *vcache;
     float* out;
@@ -603,9 +607,11 @@ struct PrefillAttnF32 {
 template <int HD>
 __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32 p) {
     typedef float floatx16 __attribute__((ext_vector_type(16)));
-    constexpr int KS = 4, NT = HD / 32, QROW = HD + 4;  // query row stride: conflict-free 16-byte reads
+    constexpr int KS = 4, NT = HD / 32;
+    constexpr int QC = 2, PC = 4;  // chains: 8 * QC dims of a score, 2 * PC keys of an output
     typedef float vrow __attribute__((ext_vector_type(NT)));
-    constexpr int STATE = NT * 16 + 2;                  // O^T, max and sum of a lane
+    constexpr int QROW = HD + 4;        // query row stride: conflict-free 16-byte reads
+    constexpr int STATE = NT * 16 + 2;  // O^T, max and sum of a lane
     constexpr int LDS_FLOATS = KS * STATE * 64 > 32 * QROW ? KS * STATE * 64 : 32 * QROW;
     __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];
 
@@ -635,14 +641,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32
 
     float4 kf[HD / 8];
     vrow vf[16];
-    auto load_k = [&](int t) __attribute__((always_inline)) {
+    // half a tile at a time (a half's registers come free in the middle of the product that uses the tile)
+    auto load_k = [&](int t, int half) __attribute__((always_inline)) {
         const unsigned at = (unsigned)min(32 * t + lq, kend - 1) * HD + 4 * h2;  // (32-bit: scalar base + offset)
 #pragma unroll
-        for (int q = 0; q < HD / 8; q++) kf[q] = *reinterpret_cast<const float4*>(kc + at + 8 * q);
+        for (int q = HD / 16 * half; q < HD / 16 * (half + 1); q++)
+            kf[q] = *reinterpret_cast<const float4*>(kc + at + 8 * q);
     };
-    auto load_v = [&](int t) __attribute__((always_inline)) {
+    auto load_v = [&](int t, int half) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
+        for (int r = 8 * half; r < 8 * half + 8; r++) {
             const unsigned key = min(32 * t + (r >> 2) * 8 + h2 * 4 + (r & 3), kend - 1);
             vf[r] = *reinterpret_cast<const vrow*>(vc + key * HD + NT * lq);
         }
@@ -657,8 +665,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32
         const int r = (tid + 256 * i) / (HD / 4), c = tid % (HD / 4), t = min(row0 + r, p.T - 1);
         qr[i] = *reinterpret_cast<const float4*>(p.q32 + ((size_t)b * p.T + t) * p.heads * HD + (size_t)head * HD + 4 * c);
     }
-    load_k(slice);
-    load_v(slice);
+    load_k(slice, 0);
+    load_k(slice, 1);
+    load_v(slice, 0);
 #pragma unroll
     for (int i = 0; i < QL; i++) {
         const int r = (tid + 256 * i) / (HD / 4), c = tid % (HD / 4);
@@ -678,9 +687,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32
         for (int r = 0; r < 16; r++) o[j][r] = 0.f;
     float m = -INFINITY, l = 0.f;
     for (int t = slice; t < ntiles; t += KS) {
-        floatx16 s;
-#pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = 0.f;
+        floatx16 s, c[2];
         // (the query values of a step are read one step ahead and no further: registers)
         const float* const qrow = &lds[lq * QROW + 4 * h2];
         float4 qv = *reinterpret_cast<const float4*>(qrow);
@@ -688,15 +695,23 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32
         for (int q = 0; q < HD / 8; q++) {
             float4 qn = qv;
             if (q + 1 < HD / 8) qn = *reinterpret_cast<const float4*>(qrow + 8 * (q + 1));
+            floatx16& x = c[q / QC & 1];
+            if (q % QC == 0)
+#pragma unroll
+                for (int r = 0; r < 16; r++) x[r] = 0.f;
             __builtin_amdgcn_sched_barrier(0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].x, qv.x, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].y, qv.y, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].z, qv.z, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].w, qv.w, s, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].x, qv.x, x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].y, qv.y, x, 0, 0, 0);
+            if (q == QC) s = c[0];
+            if (q > QC && q % QC == 0) s += c[(q / QC & 1) ^ 1];
+            x = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].z, qv.z, x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[q].w, qv.w, x, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
+            if (q == HD / 16) load_v(t, 1);
             qv = qn;
         }
-        load_k(t + KS);
+        s += c[(HD / 8 / QC - 1) & 1];
+        load_k(t + KS, 0);
         const int k0 = 32 * t;
         if (k0 + 31 > p.p0 + row0) {  // tiles past the first row's own key (row0 + 31 >= T lies there too)
 #pragma unroll
@@ -719,18 +734,34 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(PrefillAttnF32
         }
         // a query whose keys in this wavefront's tiles are all masked so far keeps m = -inf: weights 0
         const float mu = (m == -INFINITY) ? 0.f : m;
-        float sum = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            s[r] = __builtin_amdgcn_exp2f(s[r] - mu);
-            sum += s[r];
+        for (int r = 0; r < 16; r++) s[r] = __builtin_amdgcn_exp2f(s[r] - mu);
+        float sum[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) sum[r] = s[r] + s[r + 8];
+#pragma unroll
+        for (int n = 4; n > 0; n /= 2)
+#pragma unroll
+            for (int r = 0; r < n; r++) sum[r] += sum[r + n];
+        l += sum_xor32(sum[0]);
+        constexpr int CHAINS = 16 / PC * NT;
+#pragma unroll
+        for (int n = 0; n < CHAINS; n++) {  // chain n: the keys of steps r0 .. r0 + PC - 1 into O^T tile j
+            const int j = n % NT, r0 = n / NT * PC;
+            floatx16& x = c[n & 1];
+#pragma unroll
+            for (int r = 0; r < 16; r++) x[r] = 0.f;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < PC; r++) {
+                x = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[r0 + r][j], s[r0 + r], x, 0, 0, 0);
+                if (r == PC / 2 - 1 && n > 0) o[(n - 1) % NT] += c[(n & 1) ^ 1];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (n == CHAINS / 2) load_k(t + KS, 1);
         }
-        l += sum_xor32(sum);
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-#pragma unroll
-            for (int j = 0; j < NT; j++) o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[r][j], s[r], o[j], 0, 0, 0);
-        load_v(t + KS);
+        o[NT - 1] += c[(CHAINS - 1) & 1];
+        load_v(t + KS, 0);
     }
 
     __syncthreads();  // the queries are read: their LDS takes the states

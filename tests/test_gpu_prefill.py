@@ -324,6 +324,30 @@ def test_row_preparation_forms_give_the_same_bits(ctx):
         np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+def test_prefill_fp32_attention_sums_in_short_chains(ctx, hd):
+    """One token repeated, zero queries: every weight is 1 and every value row the same, so the last row's
+    attention output is the value row itself (what a one-token prompt returns) up to the roundings of its
+    sum.  A sum of n equal rows loses at most n / 2 units of 2^-24: chains of 8 keys, four of them from each
+    32-key tile of a wavefront's quarter one after another; and three merges, the division, its rounding."""
+    T = 2047
+    cfg = C.Qwen3Config(dim=256, hidden_dim=64, layer_count=1, head_count=256 // hd, kv_head_count=256 // hd,
+                        vocab_size=256, seq_len=T + 1, head_size=hd, qk_norm_mode=C.QK_NORM_PER_HEAD)
+    sd = _one_product_weights(cfg, seed=5)
+    sd["model.layers.0.self_attn.q_proj.weight"] = np.zeros((cfg.q_dim, cfg.dim), np.float32)
+    token, out = 17, {}
+    with Qwen3(cfg, sd, ctx) as m:
+        for n in (1, 40, 700, T):
+            m.model.reset()
+            m.model.set_prompt(np.full(n, token))
+            m.model.prefill()
+            out[n] = np.delete(m.model.hidden()[0].astype(np.float64), token)  # (that dim holds the embedding)
+        assert m.model.prefill_by_steps() == 0
+    for n in (40, 700, T):
+        err = np.abs(out[n] / out[1] - 1).max()
+        assert err <= (8 / 2 + 4 * np.ceil(n / 128) / 2 + 5) * 2.0 ** -24, (n, err * 2.0 ** 24)
+
+
 def test_prefill_fp32_c3_prompt_vs_oracle(ctx):
     """BASELINE config 3 (Qwen3-0.6B shape, fp32, q_dim 2048 != dim): the 128-token prompt through
     the fp32 batched prefill, then 8 greedy steps, against the FP32 oracle's batched prompt pass
