@@ -15,18 +15,22 @@
 // reaches top_p.  With p* the smallest kept value, that is every value > p* plus the first c
 // (by index) of the values == p*; p* is the largest key t with sum(p >= t) >= top_p.  It is found
 // on the 64-bit patterns of the probabilities (non-negative doubles order as their bit patterns):
-//  * one pass over the row adds the values into 1,024 buckets by exponent and the first four mantissa
-//    bits (64 octaves below 1; what lies lower is below the fixed point's unit and never holds p*), LDS
-//    per chunk, then the row's buckets with device-scope atomics; the last chunk to finish (an arrival
-//    counter) picks the bucket whose range holds p* and clears the row's buckets for the next draw;
+//  * one pass over the row adds the values into 1,024 buckets of equal width in the bit pattern between the
+//    row's least and largest value, or by exponent and the first four mantissa bits where they lie further
+//    apart than that covers (64 octaves below 1; what lies lower is below the fixed point's unit and never
+//    holds p*), LDS per chunk, then the row's buckets with device-scope atomics; the last chunk to finish
+//    (an arrival counter) picks the bucket whose range holds p* and clears the row's buckets for the next
+//    draw;
 //  * one pass copies that bucket's values, in index order, and sums what lies above it per chunk;
-//  * the block that draws finishes the search on the copied values alone (a radix descent over the
-//    remaining 48 bits, 8 at a time, ending early once one value is left).
-// 8 x 151,936 values: 55 us a draw (draw 20, buckets 14, exponentials 11, copy 6.5, maximum 4: launches and
-// the serial chain of the drawing block, not the 4.9 MB of logits), against 124 with eight 8-bit passes over the whole row, whose
-// first digits separate next to nothing.  Bucket sums are 2^-60 fixed point in u64, so the atomics are
-// exact and associative (the result does not depend on arrival order); the kept set agrees with the
-// reference's sequential double sums except when top_p lies within ~1e-13 of a partial sum.
+//  * the block that draws finishes the search on the copied values alone (a radix descent over the bucket's
+//    bits, at most 48 and 8 at a time, ending early once one value is left).
+// 8 x 151,936 values: 56 us a draw, against 124 with eight 8-bit passes over the whole row, whose first
+// digits separate next to nothing.  Buckets by exponent and mantissa alone put a whole row of equal or
+// nearly equal logits into one bucket, for the drawing block to go over digit by digit: one row of 151,936
+// equal logits took 1,662 us (deviation 0.001: 256; rounded to whole numbers: 468), 33, 40 and 62 now, and 97,
+// 76 and 77 with the eight passes.  Bucket sums are 2^-60 fixed point in u64, so the atomics are exact and
+// associative (the result does not depend on arrival order); the kept set agrees with the reference's
+// sequential double sums except when top_p lies within ~1e-13 of a partial sum.
 //
 // The draw mirrors the reference's loop `cumulative += probs[i]; if (r < cumulative) return i`:
 // chunk masses locate the chunk whose interval holds r, then per-thread sums of contiguous index
@@ -50,11 +54,13 @@ struct Ws {
     double* pmax;               // [rows][kBlocks]
     double* psum;
     double* pemax;
+    double* pemin;
     double* psum2;
     double* pmass;
     unsigned long long* gsum;   // [rows][kBins] fixed-point bucket sums of the row (zero between draws)
     unsigned* arrived;          // [rows] chunks done with the bucket pass (zero between draws)
-    unsigned long long* sel;    // [rows][2]: bucket of p* (or -1: everything is kept), fixed-point sum above it
+    unsigned long long* sel;    // [rows][4]: the bucket of p*: least key (or -1: everything is kept), fixed-
+                                // point sum above it, bits of its width
     unsigned long long* cand;   // [rows][V] bit patterns of the bucket's values, each chunk's at its own start
     unsigned* ncand;            // [rows][kBlocks]
 };
@@ -77,9 +83,10 @@ Ws carve(void* base, int rows, int V, size_t* total, size_t* zero_bytes) {
     w.pmax = (double*)take((size_t)rows * kBlocks * 8);
     w.psum = (double*)take((size_t)rows * kBlocks * 8);
     w.pemax = (double*)take((size_t)rows * kBlocks * 8);
+    w.pemin = (double*)take((size_t)rows * kBlocks * 8);
     w.psum2 = (double*)take((size_t)rows * kBlocks * 8);
     w.pmass = (double*)take((size_t)rows * kBlocks * 8);
-    w.sel = (unsigned long long*)take((size_t)rows * 2 * 8);
+    w.sel = (unsigned long long*)take((size_t)rows * 4 * 8);
     w.cand = (unsigned long long*)take((size_t)rows * V * 8);
     w.ncand = (unsigned*)take((size_t)rows * kBlocks * 4);
     if (total) *total = off;
@@ -155,6 +162,7 @@ __device__ inline T block_incl_scan(T v, T* red) {
 }
 // combine one row's 64 chunk partials (every thread gets the value; same order in every block)
 __device__ inline double row_max(const double* p) { return wave_max_d(p[threadIdx.x & 63]); }
+__device__ inline double row_max_neg(const double* p) { return wave_max_d(-p[threadIdx.x & 63]); }
 __device__ inline double row_sum(const double* p) { return wave_sum_d(p[threadIdx.x & 63]); }
 
 __device__ inline void chunk_of(int V, int blk, int* c0, int* c1) {
@@ -180,12 +188,12 @@ __global__ __launch_bounds__(kThreads) void smp_max_kernel(Args a) {
 // 2. exponentials: sampleToken's exp(x - max), or the softmax-ignoring-zero of the model's sample
 //    function (a value equal to 0 stays 0; the maximum itself gets exp(epsilon))
 __global__ __launch_bounds__(kThreads) void smp_exp_kernel(Args a) {
-    __shared__ double red[kWaves];
+    __shared__ double red[3 * kWaves];
     const int blk = blockIdx.x, b = blockIdx.y;
     int c0, c1;
     chunk_of(a.V, blk, &c0, &c1);
     const double M = row_max(a.w.pmax + b * kBlocks);
-    double s = 0.0, emax = 0.0;
+    double s = 0.0, emax = 0.0, emin = INFINITY;
     double* buf = a.w.buf + (size_t)b * a.V;
     for (int i = c0 + threadIdx.x; i < c1; i += kThreads) {
         const double y = scaled(a, b, i);
@@ -199,10 +207,26 @@ __global__ __launch_bounds__(kThreads) void smp_exp_kernel(Args a) {
         buf[i] = e;
         s += e;
         emax = fmax(emax, e);
+        emin = fmin(emin, e);
     }
-    s = block_sum_d(s, red);
-    emax = block_max_d(emax, red);
+    // the three block reductions under one barrier, for thread 0 alone
+    s = wave_sum_d(s);
+    emax = wave_max_d(emax);
+    emin = -wave_max_d(-emin);
+    if ((threadIdx.x & 63) == 0) {
+        const int w = threadIdx.x >> 6;
+        red[w] = s;
+        red[kWaves + w] = emax;
+        red[2 * kWaves + w] = emin;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
+        for (int w = 1; w < kWaves; w++) {
+            s += red[w];
+            emax = fmax(emax, red[kWaves + w]);
+            emin = fmin(emin, red[2 * kWaves + w]);
+        }
+        a.w.pemin[b * kBlocks + blk] = emin;
         a.w.psum[b * kBlocks + blk] = s;
         a.w.pemax[b * kBlocks + blk] = emax;
     }
@@ -232,11 +256,23 @@ __device__ inline double denom(const Args& a, int b) {
     return row_sum((a.mode == AR_SAMPLE_TOKEN ? a.w.psum : a.w.psum2) + b * kBlocks);
 }
 
-// Bucket of a probability in [0, 1]: exponent and four mantissa bits, 1.0 in the last one, everything
-// under 2^-63.9 in the first.
-__device__ inline int bucket_of(double p) {
-    const int d = (int)((unsigned long long)__double_as_longlong(p) >> 48) - (0x3FF0 - (kBins - 1));
-    return min(max(d, 0), kBins - 1);
+// Buckets of a row's probabilities: (key - base) >> bits, keys under base in the first.
+struct Buckets {
+    unsigned long long base;
+    int bits;
+    __device__ int of(unsigned long long key) const {
+        return key <= base ? 0 : (int)min((key - base) >> bits, (unsigned long long)(kBins - 1));
+    }
+};
+
+// Width 2^bits and first key, from the row's least and largest probability (e / D is monotone in e).
+__device__ inline Buckets buckets_of(const Args& a, int b, double D) {
+    const double* const pe = a.w.pemin + b * kBlocks;
+    const unsigned long long lo = (unsigned long long)__double_as_longlong(-row_max_neg(pe) / D),
+                             hi = (unsigned long long)__double_as_longlong(row_max(a.w.pemax + b * kBlocks) / D);
+    const int bits = hi > lo ? max(0, 54 - __clzll((long long)(hi - lo))) : 0;
+    if (bits > 48) return Buckets{(unsigned long long)(0x3FF0 - (kBins - 1)) << 48, 48};  // (1.0 in the last)
+    return Buckets{lo, bits};
 }
 
 // 4. nucleus search, the whole row: probabilities (written back over the exponentials) into the buckets;
@@ -251,12 +287,13 @@ __global__ __launch_bounds__(kThreads) void smp_bucket_kernel(Args a) {
     int c0, c1;
     chunk_of(a.V, blk, &c0, &c1);
     const double D = denom(a, b);
+    const Buckets bk = buckets_of(a, b, D);
     double* buf = a.w.buf + (size_t)b * a.V;
     for (int i = c0 + t; i < c1; i += kThreads) {
         const double p = buf[i] / D;
         buf[i] = p;
         const unsigned long long f = (unsigned long long)(p * kFix);
-        if (f) atomicAdd(&sm[bucket_of(p)], f);
+        if (f) atomicAdd(&sm[bk.of((unsigned long long)__double_as_longlong(p))], f);
     }
     __syncthreads();
     unsigned long long* g = a.w.gsum + (size_t)b * kBins + t;
@@ -277,13 +314,14 @@ __global__ __launch_bounds__(kThreads) void smp_bucket_kernel(Args a) {
     const unsigned long long mine = __hip_atomic_load(g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(g, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long incl = block_incl_scan(mine, red);
-    unsigned long long* sel = a.w.sel + b * 2;
+    unsigned long long* sel = a.w.sel + b * 4;
     // the whole row may sum to less than top_p (the reference then keeps every value): no bucket
     if (t == kThreads - 1 && (incl < a.target || incl == 0)) sel[0] = ~0ull;
     const unsigned long long before = incl - mine;
     if (mine && incl >= a.target && (before < a.target || before == 0)) {
-        sel[0] = (unsigned long long)(kBins - 1 - t);
+        sel[0] = bk.base + ((unsigned long long)(kBins - 1 - t) << bk.bits);
         sel[1] = before;
+        sel[2] = bk.bits;
     }
 }
 
@@ -294,9 +332,9 @@ __global__ __launch_bounds__(kThreads) void smp_cand_kernel(Args a) {
     const int blk = blockIdx.x, b = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
     int c0, c1;
     chunk_of(a.V, blk, &c0, &c1);
-    const unsigned long long sel = a.w.sel[b * 2];
-    const bool cut = sel != ~0ull;
-    const int bin = cut ? (int)sel : -1;  // (no cut: everything lies above)
+    const unsigned long long base = a.w.sel[b * 4];
+    const bool cut = base != ~0ull;
+    const int bits = cut ? (int)a.w.sel[b * 4 + 2] : 0;
     const double* buf = a.w.buf + (size_t)b * a.V;
     unsigned long long* cand = a.w.cand + (size_t)b * a.V + c0;
     double s = 0.0;
@@ -304,9 +342,9 @@ __global__ __launch_bounds__(kThreads) void smp_cand_kernel(Args a) {
     for (int i0 = c0; i0 < c1; i0 += kThreads) {
         const int i = i0 + t;
         const double p = i < c1 ? buf[i] : 0.0;
-        const int d = bucket_of(p);
-        if (i < c1 && (!cut || d > bin)) s += p;
-        const bool in = i < c1 && cut && d == bin;
+        const unsigned long long key = (unsigned long long)__double_as_longlong(p);
+        const bool in = i < c1 && cut && key >= base && (key - base) >> bits == 0;
+        if (i < c1 && (!cut || (key >= base && !in))) s += p;  // (no cut: everything lies above)
         const unsigned long long hits = __ballot(in);
         if (lane == 0) wcnt[wave] = __popcll(hits);
         __syncthreads();
@@ -315,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void smp_cand_kernel(Args a) {
             if (w < wave) at += wcnt[w];
             n += wcnt[w];
         }
-        if (in) cand[at + __popcll(hits & ((1ull << lane) - 1))] = (unsigned long long)__double_as_longlong(p);
+        if (in) cand[at + __popcll(hits & ((1ull << lane) - 1))] = key;
         __syncthreads();
     }
     s = block_sum_d(s, red);
@@ -362,52 +400,191 @@ __device__ inline double kept(const Nucleus& n, double q, unsigned long long* ra
 
 // LDS of the drawing block's end of the nucleus search
 struct SearchLds {
-    unsigned long long key[kCandLds];  // the bucket's values (when they fit), in index order
+    union {
+        unsigned long long key[kCandLds];  // the bucket's values (when they fit), in index order
+        struct {                           // ranges of a bucket that does not fit
+            unsigned long long sum[kBins], lo[kBins], hi[kBins];
+            unsigned cnt[kBins];
+        } range;
+    };
     unsigned long long sum[256];
     unsigned cnt[256];
     unsigned off[kBlocks + 1];         // first value of each chunk in that order
     unsigned long long ties[kBlocks];  // values == p* in the chunks before each chunk
     double mass[kBlocks];              // kept mass of each chunk
-    unsigned long long prefix, above, pstar, take;
+    unsigned long long prefix, above, pstar, take;  // prefix: p* - the bucket's least key, as far as known
+    unsigned long long lo, hi;
     unsigned left;
+    int pick;
 };
 
-// p*, the ties kept, and the kept mass of every chunk (L.mass), by the whole block.
-__device__ Nucleus finish_search(const Args& a, int b, SearchLds& L) {
+// A bucket of more than kCandLds values, L.lo .. L.hi and not all equal (many equal values among others): cut
+// down to the values that may be p*, its surroundings added to the chunks' mass.  Each round spreads the keys
+// over 1,024 ranges of equal width and goes on with the span (least to largest key) of the one that holds p*,
+// until its values are equal or fit L.key.  A thread adds up its run of values of one range before it touches
+// LDS: atomics of a wavefront on one address go one after another.  Then one pass sums the keys above per
+// chunk and moves the rest to the front of the chunk's copies (equal values: counts them).  L.ties: what
+// is left of each chunk.  Bound by one CU's read of the copies: some 30 us a pass over 151,936 values.
+__device__ void thin_bucket(const Args& a, int b, SearchLds& L, unsigned long long* red) {
+    constexpr int U = 8;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const unsigned long long bin = a.w.sel[b * 2];
-    if (t < kBlocks) L.mass[t] = a.w.pmass[b * kBlocks + t];
-    if (bin == ~0ull) {
-        __syncthreads();
-        return Nucleus{false, 0, 0};
-    }
-    if (t < kBlocks) {
-        const unsigned c = a.w.ncand[b * kBlocks + t], incl = wave_incl_scan(c);
-        L.off[t + 1] = incl;
-        if (t == 0) L.off[0] = 0;
-    }
-    if (t == 0) {
-        L.prefix = (unsigned long long)(0x3FF0 - (kBins - 1) + (int)bin) << 48;
-        L.above = a.w.sel[b * 2 + 1];
-    }
-    __syncthreads();
-    const unsigned n = L.off[kBlocks];
-    const bool in_lds = n <= (unsigned)kCandLds;
-    // chunk by chunk, a wavefront each: f(chunk, value index, key) for every copied value
-    auto each = [&](auto&& f) {
+    unsigned long long* const cand = a.w.cand + (size_t)b * a.V;
+    // every value of this wavefront's chunks, in index order, in groups of 64 (0 past the end: below every
+    // key), eight of them loaded together
+    auto each = [&](auto&& group, auto&& chunk_end) {
         for (int c = wave; c < kBlocks; c += kWaves) {
             int c0, c1;
             chunk_of(a.V, c, &c0, &c1);
-            const unsigned long long* src = a.w.cand + (size_t)b * a.V + c0;
+            const unsigned m = L.off[c + 1] - L.off[c];
+            for (unsigned i0 = 0; i0 < m; i0 += 64 * U) {
+                unsigned long long k[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) k[u] = cand[c0 + min(i0 + 64 * u + lane, m - 1)];
+#pragma unroll
+                for (int u = 0; u < U; u++) group(c0, i0 + 64 * u + lane < m ? k[u] : 0ull);
+            }
+            chunk_end(c);
+        }
+    };
+    unsigned long long lo = L.lo, hi = L.hi;
+    for (int round = 0; round < 5; round++) {  // (48 bits, ten with every round)
+        const int sh = max(0, 54 - __clzll((long long)(hi - lo)));
+        __syncthreads();
+        L.range.sum[t] = 0;
+        L.range.lo[t] = ~0ull;
+        L.range.hi[t] = 0;
+        L.range.cnt[t] = 0;
+        if (t == 0) L.pick = kBins;
+        __syncthreads();
+        int run = -1;
+        unsigned n = 0;
+        unsigned long long s = 0, mn = ~0ull, mx = 0;
+        auto flush = [&]() {
+            if (run < 0) return;
+            atomicAdd(&L.range.cnt[run], n);
+            atomicAdd(&L.range.sum[run], s);
+            atomicMin(&L.range.lo[run], mn);
+            atomicMax(&L.range.hi[run], mx);
+        };
+        each([&](int, unsigned long long key) {
+            if (key < lo || key > hi) return;
+            const int d = (int)((key - lo) >> sh);
+            if (d != run) {
+                flush();
+                run = d;
+                n = 0;
+                s = 0;
+                mn = ~0ull;
+                mx = 0;
+            }
+            n++;
+            s += (unsigned long long)(__longlong_as_double((long long)key) * kFix);
+            mn = min(mn, key);
+            mx = max(mx, key);
+        }, [](int) {});
+        flush();
+        __syncthreads();
+        const int d = kBins - 1 - t;  // an inclusive scan in thread order sums the ranges from the top
+        const unsigned long long mine = L.range.sum[d], incl = block_incl_scan(mine, red);
+        if (L.range.cnt[d] && L.above + incl >= a.target) atomicMin(&L.pick, t);
+        __syncthreads();
+        if (t == L.pick) {  // (the bucket holds p*: one does)
+            L.lo = L.range.lo[d];
+            L.hi = L.range.hi[d];
+            L.left = L.range.cnt[d];
+            L.above += incl - mine;
+        }
+        __syncthreads();
+        lo = L.lo;
+        hi = L.hi;
+        if (lo >= hi || L.left <= (unsigned)kCandLds) break;
+    }
+    const bool equal = L.left > (unsigned)kCandLds;
+    double s = 0.0;
+    unsigned n = 0;
+    each([&](int c0, unsigned long long key) {
+        if (key > hi) s += __longlong_as_double((long long)key);
+        const bool in = key >= lo && key <= hi;
+        const unsigned long long hits = __ballot(in);
+        // (at or before the place it was read from, and behind what is still to be read)
+        if (!equal && in) cand[c0 + n + __popcll(hits & ((1ull << lane) - 1))] = key;
+        n += __popcll(hits);
+    }, [&](int c) {
+        const double total = wave_sum_d(s);
+        if (lane == 0) {
+            L.mass[c] += total;
+            L.ties[c] = n;
+        }
+        s = 0.0;
+        n = 0;
+    });
+    __syncthreads();
+    if (!equal && t < kBlocks) L.off[t + 1] = (unsigned)wave_incl_scan(L.ties[t]);
+    __syncthreads();
+}
+
+// p*, the ties kept, and the kept mass of every chunk (L.mass), by the whole block.
+__device__ Nucleus finish_search(const Args& a, int b, SearchLds& L, unsigned long long* red) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    unsigned long long base = a.w.sel[b * 4];
+    if (t < kBlocks) L.mass[t] = a.w.pmass[b * kBlocks + t];
+    if (base == ~0ull) {
+        __syncthreads();
+        return Nucleus{false, 0, 0};
+    }
+    int bits = (int)a.w.sel[b * 4 + 2];  // keys base .. base + 2^bits - 1
+    if (t < kBlocks) {
+        const unsigned c = a.w.ncand[b * kBlocks + t], incl = wave_incl_scan(c);
+        L.off[t + 1] = incl;
+        L.ties[t] = c;
+        if (t == 0) L.off[0] = 0;
+        if (t == kBlocks - 1) L.left = incl;
+    }
+    if (t == 0) {
+        L.prefix = 0;
+        L.above = a.w.sel[b * 4 + 1];
+        L.lo = base;
+        L.hi = base + ((1ull << bits) - 1);
+    }
+    __syncthreads();
+    // values == p* kept, of the L.left there are
+    auto set_take = [&]() {
+        const unsigned long long pf = (unsigned long long)(__longlong_as_double((long long)L.pstar) * kFix);
+        unsigned long long take = 1;
+        if (a.target > L.above) take = pf ? (a.target - L.above + pf - 1) / pf : L.left;
+        L.take = take < 1 ? 1 : (take > L.left ? L.left : take);
+    };
+    if (bits && L.left > (unsigned)kCandLds) thin_bucket(a, b, L, red);
+    base = L.lo;
+    bits = 64 - (L.hi > base ? __clzll((long long)(L.hi - base)) : 64);
+    if (L.left > (unsigned)kCandLds) {
+        // equal values: the first `take` by index, chunk by chunk
+        if (t == 0) {
+            L.pstar = base;
+            set_take();
+        }
+        __syncthreads();
+        const Nucleus nu{true, L.pstar, L.take};
+        if (t < kBlocks) {
+            const unsigned long long v = L.ties[t], before = wave_incl_scan(v) - v;
+            const unsigned long long k = nu.take > before ? min(nu.take - before, v) : 0ull;
+            L.ties[t] = before;
+            L.mass[t] += (double)k * __longlong_as_double((long long)nu.pstar);
+        }
+        __syncthreads();
+        return nu;
+    }
+    // chunk by chunk, a wavefront each: f(chunk, key, live) for every copied value
+    auto each = [&](auto&& f) {
+        for (int c = wave; c < kBlocks; c += kWaves) {
             const unsigned o = L.off[c], m = L.off[c + 1] - o;
             for (unsigned i0 = 0; i0 < m; i0 += 64) {
-                const unsigned i = i0 + lane;
-                const bool live = i < m;
-                f(c, o + i, live ? (in_lds ? L.key[o + i] : src[i]) : 0ull, live);
+                const bool live = i0 + lane < m;
+                f(c, live ? L.key[o + i0 + lane] : 0ull, live);
             }
         }
     };
-    if (in_lds) {  // 16 lanes a chunk: usually one load each
+    {  // 16 lanes a chunk: usually one load each
         int c0, c1;
         const int c = t / (kThreads / kBlocks);
         chunk_of(a.V, c, &c0, &c1);
@@ -415,17 +592,27 @@ __device__ Nucleus finish_search(const Args& a, int b, SearchLds& L) {
         for (unsigned i = t % (kThreads / kBlocks); i < m; i += kThreads / kBlocks)
             L.key[o + i] = a.w.cand[(size_t)b * a.V + c0 + i];
     }
-    // radix descent: the highest digit d with above + sum(digits >= d) >= target at each level
-    for (int shift = 40;; shift -= 8) {
+    // radix descent over key - base: the highest digit d with above + sum(digits >= d) >= target at each level
+    for (int left = bits;;) {  // bits that are still open
+        if (left == 0 || L.left == 1) {
+            // every value left has the prefix's bits: one value, or equal ones
+            __syncthreads();
+            const unsigned long long pre = L.prefix >> left;
+            each([&](int, unsigned long long key, bool live) {
+                if (live && (key - base) >> left == pre) L.pstar = key;
+            });
+            break;
+        }
+        const int width = min(left, 8), shift = left - width;
         if (t < 256) {
             L.cnt[t] = 0;
             L.sum[t] = 0;
         }
         __syncthreads();
-        const unsigned long long want = L.prefix >> (shift + 8), above = L.above;
-        each([&](int, unsigned, unsigned long long key, bool live) {
-            if (live && (key >> (shift + 8)) == want) {
-                const int d = (int)((key >> shift) & 255);
+        const unsigned long long want = L.prefix >> left, above = L.above;
+        each([&](int, unsigned long long key, bool live) {
+            if (live && (key - base) >> left == want) {
+                const int d = (int)(((key - base) >> shift) & ((1u << width) - 1));
                 atomicAdd(&L.cnt[d], 1u);
                 atomicAdd(&L.sum[d], (unsigned long long)(__longlong_as_double((long long)key) * kFix));
             }
@@ -455,29 +642,17 @@ __device__ Nucleus finish_search(const Args& a, int b, SearchLds& L) {
             }
         }
         __syncthreads();
-        if (shift == 0 || L.left == 1) {
-            // every value left has the prefix's bits: one value, or equal ones
-            const unsigned long long pre = L.prefix >> shift;
-            each([&](int, unsigned, unsigned long long key, bool live) {
-                if (live && (key >> shift) == pre) L.pstar = key;
-            });
-            break;
-        }
+        left = shift;
     }
     __syncthreads();
-    if (t == 0) {
-        const unsigned long long pf = (unsigned long long)(__longlong_as_double((long long)L.pstar) * kFix);
-        unsigned long long take = 1;  // values == p* kept
-        if (a.target > L.above) take = pf ? (a.target - L.above + pf - 1) / pf : L.left;
-        L.take = take < 1 ? 1 : (take > L.left ? L.left : take);
-    }
+    if (t == 0) set_take();
     __syncthreads();
-    Nucleus nu{true, L.pstar, L.take};
+    const Nucleus nu{true, L.pstar, L.take};
     // ties before each chunk, then the kept mass of the bucket's values per chunk (lane sums in index
     // order, then the lanes): added to the mass above the bucket
     for (int c = wave; c < kBlocks; c += kWaves)
         if (lane == 0) L.ties[c] = 0;
-    each([&](int c, unsigned, unsigned long long key, bool live) {
+    each([&](int c, unsigned long long key, bool live) {
         const unsigned long long hits = __ballot(live && key == nu.pstar);
         if (lane == 0) L.ties[c] += __popcll(hits);
     });
@@ -496,7 +671,7 @@ __device__ Nucleus finish_search(const Args& a, int b, SearchLds& L) {
         if (lane == 0) L.mass[cur] += total;
         s = 0.0;
     };
-    each([&](int c, unsigned, unsigned long long key, bool live) {
+    each([&](int c, unsigned long long key, bool live) {
         if (c != cur) {
             flush();
             cur = c;
@@ -537,7 +712,7 @@ __global__ __launch_bounds__(kThreads) void smp_draw_kernel(Args a) {
     // AutoregressiveModel.next applies its sample function (AutoregressiveModel.java:295-308).
     if (a.state && a.state[2] < a.state[1]) return;
     const double D = a.topp ? 1.0 : denom(a, b);  // (the nucleus search left probabilities in buf)
-    const Nucleus n = a.topp ? finish_search(a, b, L) : Nucleus{false, 0, 0};
+    const Nucleus n = a.topp ? finish_search(a, b, L, ured) : Nucleus{false, 0, 0};
     if (t < 64) {
         // chunk masses in index order; the first chunk whose running total exceeds r
         const double pm = a.topp ? L.mass[lane] : a.w.pmass[b * kBlocks + lane];

@@ -8,6 +8,7 @@ intervals (the device groups its partial sums differently, ~1e-16; the nucleus c
 exactly after every call (one nextDouble per sampled token, none for greedy temperatures).
 """
 import dataclasses
+import time
 
 import numpy as np
 import pytest
@@ -103,6 +104,48 @@ def test_sample_op_nucleus_buckets(ctx, n, top_p):
     logits[3] = rng.permutation(np.linspace(-4.0, 4.0, n))
     near, _ = _run_op(ctx, logits, hw.SAMPLE_TOKEN, 0.9, top_p, seeds=[7, 8, 9, 10], calls=4)
     assert near <= 1
+
+
+@pytest.mark.parametrize("n,top_p", [(4201, 0.5), (32001, 0.9), (151936, 0.3), (151936, 0.97)])
+def test_sample_op_nucleus_in_a_crowded_bucket(ctx, n, top_p):
+    """More values around the cut than the drawing block holds in LDS: every value equal; nearly equal ones
+    (one round of ranges); half of them equal between nearly equal ones (the range of the equal ones
+    alone overflows LDS); equal ones with a few a unit of the last place away.  (n * top_p is not whole:
+    where it is, top_p equals a partial sum of the equal row, and the 2^-60 fixed point and the oracle's
+    sequential sum, both within 1e-13 of it, may fall on different sides.)"""
+    print(f"[sample crowded] n={n} top_p={top_p}", flush=True)
+    rng = np.random.default_rng(n)
+    logits = np.zeros((4, n), np.float32)
+    logits[1] = rng.normal(0.0, 0.001, n)
+    logits[2] = np.where(rng.random(n) < 0.5, 0.0, rng.normal(0.0, 0.001, n))
+    logits[3] = 1.0
+    logits[3, rng.integers(0, n, 500)] = np.nextafter(np.float32(1.0), np.float32(2.0))
+    logits[3, rng.integers(0, n, 500)] = np.nextafter(np.float32(1.0), np.float32(0.0))
+    near, _ = _run_op(ctx, logits, hw.SAMPLE_TOKEN, 1.0, top_p, seeds=[21, 22, 23, 24], calls=4)
+    assert near <= 1
+
+
+def test_sample_op_equal_logits_take_no_multiple_of_the_time(ctx):
+    """Equal logits put the whole row into one bucket of the nucleus search; the draw must not go over them
+    once per digit of the search (an ordinary row's time without; 40 times that with a pass, and its atomics
+    on one address, per digit)."""
+    n, best = 151936, {}
+    out, st = ctx.allocate(4), ctx.to_device(np.array([hw.java_random_state(1)], dtype=np.uint64))
+    rows = {"spread": np.random.default_rng(1).normal(0.0, 2.0, n), "equal": np.zeros(n)}
+    for name, row in rows.items():
+        lg, times = ctx.to_device(row.astype(np.float32)), []
+        for _ in range(12):
+            ctx.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(4):
+                ctx.sample(lg, 1, n, hw.SAMPLE_TOKEN, 1.0, 0.9, st, out)
+            ctx.synchronize()
+            times.append(time.perf_counter() - t0)
+        best[name] = min(times)
+        lg.free()
+    out.free()
+    st.free()
+    assert best["equal"] <= 10 * best["spread"], best
 
 
 @pytest.mark.parametrize("mode,temperature", [(hw.SAMPLE_MODEL, 0.0), (hw.SAMPLE_TOKEN, 0.0),
