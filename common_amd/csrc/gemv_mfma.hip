@@ -1,4 +1,4 @@
-// Batched decode GEMV on the MFMA units: bf16 weights, 3..16 sequences.
+// Batched decode GEMV on the MFMA units: bf16 weights, 3..8 sequences.
 //
 // Same contract as the batch-1/2 GEMV (gemv_impl.h): the reference's dense -> matmul/weightedSum
 // (domain/graph/.../LayerFeatures.java:785-830, compute/algebra/.../MatrixFeatures.java:182-337)
@@ -17,9 +17,9 @@
 //
 // A block's wavefronts split the k-steps of a tile of weight rows and sum their 16 x 16 partial tiles
 // through LDS in a fixed order.  Two forms:
-//  * packed (up to 8 sequences, up to 16 k-steps per wavefront: cols <= 4096): one block per CU loops over
+//  * packed (up to 16 k-steps per wavefront: cols <= 4096, and at least as many tiles as CUs): one block per CU loops over
 //    tiles with the input planes in registers (see gemv_mfma_pack_kernel);
-//  * streaming (wider inputs, or fewer tiles than CUs): one tile per 16-wavefront block; each
+//  * streaming (the rest): one tile per 16-wavefront block; each
 //    chunk of k-steps issues its weight and input loads together, and the next chunk's loads are in
 //    flight while the current chunk is converted and multiplied.
 #include <algorithm>
@@ -158,7 +158,7 @@ struct Finish {
     }
 };
 
-// Up to 8 sequences: one MFMA per k-step carries both planes, lanes 0-7 of each 16-lane row the hi plane of
+// One MFMA per k-step carries both planes, lanes 0-7 of each 16-lane row the hi plane of
 // sequences 0-7 and lanes 8-15 the lo plane, so columns b and b + 8 of the result add up to sequence b's
 // products (half the MFMAs and half the plane registers of one MFMA per plane).  A tile is 16 weight
 // rows; for SwiGLU 8 gate rows and the same 8 up rows.
@@ -166,10 +166,13 @@ struct Finish {
 // tiles are always in flight (register sets, two to four: some 100 KB per CU), across the tile's one barrier, which waits for LDS only
 // (a barrier that waits for the loads too leaves the CU without any request once per tile).  Four
 // wavefronts finish a tile while the others go on.
-// 9,728 x 2,560 SwiGLU, 8 sequences: 26 us a call, 34 with one MFMA per plane, whole 16 + 16-row tiles (608
-// on 256 CUs: 2.4 rounds) and a full barrier; in a decode step of the 4B shape, weights cold in HBM: QKV
-// (6,144 x 2,560) 15.7 -> 13.7 us, 16,896-row head 31 -> 24.  Bound by HBM and, with few tiles per CU, by
-// the first loads' latency and the last round.  8-row tiles for the other epilogues too (QKV in one and a
+// In a decode step of the 4B shape, weights cold in HBM: QKV (6,144 x 2,560) 15.7 -> 13.7 us, 16,896-row
+// head 31 -> 24, against one MFMA per plane, whole 16 + 16-row tiles and a full barrier.  Bound by HBM and, with
+// few tiles per CU, by the first loads' latency and the last round.  Repeated calls on one matrix, which
+// then stays in the last-level cache: 9,728 x 2,560 SwiGLU, 8 sequences, 34 -> 26 us (608 tiles on 256 CUs were
+// 2.4 rounds).  Narrow inputs have instances of one and two k-steps: three loads a tile where one is needed
+// cost more than the tile (8,192 x 256 SwiGLU, 8 sequences: 7.9 us with three, 5.5 with one; inputs of fewer than
+// eight k-steps on the streaming form, a block per tile: 32,000 x 224 19.2 us, 6.1 here).  8-row tiles for the other epilogues too (QKV in one and a
 // half rounds instead of two) measured slower: 14.7 us, twice the barriers for the same bytes.
 template <int EPI, int KS>
 __global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv::Params p, int tiles) {
@@ -181,6 +184,7 @@ __global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15,
               q = lane >> 4, seq = r & 7;
     const int nsteps = p.cols / 32, s0 = nsteps * w / NW, ns = nsteps * (w + 1) / NW - s0;  // KS - 2 <= ns <= KS
+    const int last = max(ns - 1, 0);  // (fewer k-steps than wavefronts: some have none, and read step s0)
     const bool live = seq < p.batch, norm = p.norm_w != nullptr;
     const int step = gridDim.x;
 
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv
         const int inc = in ? 32 : 0;
 #pragma unroll
         for (int i = 0; i < KS; i++)  // (steps past ns repeat the last one; never multiplied)
-            wv[set][i] = *reinterpret_cast<const u32x4*>(src + (i < KS - 2 ? i : min(i, ns - 1)) * inc);
+            wv[set][i] = *reinterpret_cast<const u32x4*>(src + (i < KS - 2 ? i : min(i, last)) * inc);
     };
     int t = blockIdx.x;
 
@@ -217,11 +221,11 @@ __global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv
         if (norm)
 #pragma unroll
             for (int i = 0; i < KS; i++)
-                xs[i] = *reinterpret_cast<const float4*>(xrow + (i < KS - 2 ? i : min(i, ns - 1)) * 32);
+                xs[i] = *reinterpret_cast<const float4*>(xrow + (i < KS - 2 ? i : min(i, last)) * 32);
         const uint16_t* const pl = (r < 8 ? p.x_hi : p.x_lo) + xo;
 #pragma unroll
         for (int i = 0; i < KS; i++)
-            pv[i] = *reinterpret_cast<const u32x4*>(pl + (i < KS - 2 ? i : min(i, ns - 1)) * 32);
+            pv[i] = *reinterpret_cast<const u32x4*>(pl + (i < KS - 2 ? i : min(i, last)) * 32);
         if (KS <= 12) {  // (registers: above 12 steps after the sums)
             load(0, t);
             load(1, t + step);
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(kPackWaves * 64, 2) void gemv_mfma_pack_kernel(gemv
         if (KS <= 12) load(1, t + step);
 #pragma unroll
         for (int i = 0; i < KS; i++) {
-            const int k = (i < KS - 2 ? i : min(i, ns - 1)) * 32;
+            const int k = (i < KS - 2 ? i : min(i, last)) * 32;
             const bool use = live && (i < KS - 2 || i < ns);
             u32x4 hi, lo;
             make_planes(load4(p.x + xo + k, use), load4(p.x + xo + k + 4, use), norm ? p.norm_w + koff + k : nullptr, ss,
@@ -359,6 +363,8 @@ void launch_pack(const gemv::Params& p, int cus, hipStream_t st) {
     const int ks = (p.cols / 32 + kPackWaves - 1) / kPackWaves;
 #define AR_PACK(K) \
     if (ks <= K) return ar_launch((gemv_mfma_pack_kernel<EPI, K>), grid, block, 0, st, p, tiles)
+    AR_PACK(1);
+    AR_PACK(2);
     AR_PACK(3);
     AR_PACK(4);
     AR_PACK(5);
@@ -507,8 +513,7 @@ int launch_epi(const gemv::Params& p, hipStream_t st) {
     // fewer tiles than CUs (the 2560-row projections at C5): one tile per 16-wavefront block spreads
     // the loads over more wavefronts (measured: O 4096 -> 2560 15.5 us streaming vs 23.7 with one block per
     // tile of 8 wavefronts).  The packed form takes up to 16 k-steps per wavefront.
-    if (p.batch <= 8 && nsteps >= kPackWaves && nsteps <= kPackWaves * kPackSteps &&
-        (NMAT == 2 ? (p.rows + 7) / 8 : tiles) >= persist) {
+    if (nsteps <= kPackWaves * kPackSteps && (NMAT == 2 ? (p.rows + 7) / 8 : tiles) >= persist) {
         launch_pack<EPI>(p, persist, st);
     } else {
         // fewer tiles than CUs and nothing that needs the whole row in one block: split k over
@@ -535,7 +540,7 @@ int launch_epi(const gemv::Params& p, hipStream_t st) {
 }  // namespace
 
 int gemv_launch_mfma(const gemv::Params& p, int epi, hipStream_t st) {
-    AR_CHECK_ARG(p.batch >= 1 && p.batch <= 16 && p.cols % 32 == 0, "MFMA GEMV: batch %d / cols %d unsupported",
+    AR_CHECK_ARG(p.batch >= 1 && p.batch <= 8 && p.cols % 32 == 0, "MFMA GEMV: batch %d / cols %d unsupported",
                  p.batch, p.cols);
     switch (epi) {
         case GEMV_EPI_STORE: return launch_epi<GEMV_EPI_STORE>(p, st);

@@ -41,6 +41,11 @@ def _rng(seed):
     (8193, 1184, 3, False, True, True),
     (4100, 3552, 7, True, False, True),
     (12289, 4096, 4, True, True, True),
+    # and narrow inputs: fewer k-steps than wavefronts, one, one or two
+    (4099, 32, 5, True, False, True),
+    (8200, 96, 8, False, True, True),
+    (12290, 224, 3, True, False, True),
+    (5003, 512, 4, True, True, True),
 ])
 def test_dense(ctx, rows, cols, batch, norm, bias, bf16):
     r = _rng(rows * 7 + cols)
@@ -70,7 +75,8 @@ def test_dense(ctx, rows, cols, batch, norm, bias, bf16):
                                                   (6144, 2048, 2, True), (9728, 2560, 8, True),
                                                   (3000, 1024, 4, False), (2048, 256, 3, True),
                                                   (2051, 416, 7, True), (4104, 3616, 5, True),
-                                                  (2049, 4096, 8, True)])
+                                                  (2049, 4096, 8, True), (2051, 32, 3, True),
+                                                  (4104, 160, 8, True), (2049, 480, 6, True)])
 def test_swiglu(ctx, rows, cols, batch, bf16):
     r = _rng(rows + cols)
     Wg = (r.standard_normal((rows, cols)) * 0.02).astype(np.float32)
