@@ -6,8 +6,8 @@
 // reference feeds one per step (engine/ml/.../AutoregressiveModel.java:295-308).
 //
 // Bound by the fp32 matrix rate (157 TFLOP/s at 2.4 GHz; 137-150 over launches of 0.1-0.4 ms, whose
-// clock is lower).  One block per CU, in whole rounds of blocks, at the tile that wastes least of them
-// (see the launch rule).
+// clock is lower).  One block per CU, in whole rounds of blocks, or several small ones, at the tile that
+// takes least time by the launch rule.
 // Epilogues: STORE (+ bias), RESIDUAL (C += product), SWIGLU (C = (A.W2^T) * silu(A.W^T)), and
 // k-slices stored separately for the consumer to add in a fixed order.
 #include <atomic>
@@ -65,21 +65,25 @@ typedef __attribute__((address_space(3))) void lds_void;
 // The small tiles take eight or four stages: their products stream the weights, cold from HBM, and two
 // stages ran the 128-row products of a 0.6B layer in 28 (gate/up) and 20 us (the others) against 24 and
 // 13; the large tiles are as fast with two.
-// MFMA busy 86-88% of a block's cycles.  A second block on the CU does not raise that and makes the
-// last round uneven (both blocks of a pair end together, the leftover blocks pair up again on the CUs
-// that end first: 1,531 x 3,072 x 1,024 SwiGLU 164 us at one block per CU, 267 us at two), so a launch
-// asks for more than half of a CU's LDS.
+// A second large block on the CU makes the last round uneven (both blocks of a pair end together, the
+// leftover blocks pair up again on the CUs that end first: 1,531 x 3,072 x 1,024 SwiGLU 164 us at one block
+// per CU, 267 us at two), so their launches ask for more than half of a CU's LDS.  The 32-row tiles of many
+// rows (CH 2) are the other way round: 32 x 64 has 512 cycles of MFMAs a k-tile, less than a load takes,
+// so two stages and one block per CU leave the matrix units waiting, and its start and stores are a fifth
+// of a short product.  With four stages, three (32 x 64) or two (32 x 128) blocks share a CU: 1,672 x
+// 4,032 x 320 79 -> 51 us, 1,900 x 1,728 x 960 104 -> 70.
 template <int MB, int WN, int CH, int EPI>
 struct F32Shape {
     static constexpr int KG = 4 / WN, NB = EPI == GEMV_EPI_SWIGLU ? 2 : 1;
     static constexpr int BM = 32 * MB, NOUT = 32 * WN, BN = NOUT * NB;  // output tile BM x NOUT, BN weight rows
     static constexpr int STAGE = (BM + BN) * BK;               // floats of one stage
-    // stages: two, or for the small tiles (CH 4) eight or four of them, up to 152 KB
-    static constexpr int ST = CH <= 2 ? 2 : 8 * STAGE <= 38 * 1024 ? 8 : 4;
+    static constexpr bool SHARE = CH <= 2 && MB == 1 && NB == 1;  // several blocks per CU
+    // stages: two, four for blocks that share a CU, or for the small tiles (CH 4) eight or four, up to 152 KB
+    static constexpr int ST = SHARE ? 4 : CH <= 2 ? 2 : 8 * STAGE <= 38 * 1024 ? 8 : 4;
     static constexpr int RED = KG > 1 ? WN * MB * NB * 1024 : 0;  // the second k-group's sums
     static constexpr int USED = (ST * STAGE > RED ? ST * STAGE : RED) * 4;
-    // more than half of a CU's 160 KB: one block per CU
-    static constexpr int LDS_BYTES = USED > 82 * 1024 ? USED : 82 * 1024;
+    // more than half of a CU's 160 KB (one block per CU), or 48 and 80 KB: three and two blocks
+    static constexpr int LDS_BYTES = SHARE || USED > 82 * 1024 ? USED : 82 * 1024;
 };
 
 template <int MB, int WN, int CH, int EPI>
@@ -251,15 +255,19 @@ int launch_t(const Params& p, hipStream_t st) {
     return AR_HIP_OK;
 }
 
-// The tile with the least time over whole rounds of one block per CU: a round of 32*MB x 32*WN tiles
-// takes their MFMA cycles over 0.87 and some 2,500 cycles of start, k-group fold and stores.  Measured
-// (us; the forms before this kernel, then the chosen tile against the next best): 1,531 x 4,096 x 1,024
-// 118, 96 x 128 in two rounds 111, 128 x 128 in two 145; 1,531 x 1,024 x 3,072 113, 96 x 64 in one round
-// 85, 64 x 128 in one 102; 1,531 x 3,072 x 1,024 SwiGLU 218, 96 x 64 in three 164, 64 x 64 in five 199;
-// 2,048 x 6,144 x 2,048 SwiGLU 954, 128 x 64 in six 799.  Below 512 rows the sums stay in four chains
+// The tile with the least time over whole rounds of blocks.  Time of a round in us: the MFMA cycles of a
+// 32*MB x 32*WN tile at what they measured (0.48 ns a cycle; 0.58 and 0.495 for the 32 x 64 and 32 x 128
+// blocks that share a CU), and the start, k-group fold and stores (1 + 2*MB; shared blocks 0.75 and 2.25, for
+// the rest of it once a launch).  Fitted over 90 shapes of 512..2,048 rows, N 512..4,096, K 256..3,072 with every
+// tile timed on each: 1% spread, and the tile chosen is 0.2% off the best of its shape on average, 5% at
+// most.  Two terms in MFMA cycles and one block per CU throughout (the rule before) chose 32 x 64 in eleven rounds
+// for 1,549 x 3,520 x 2,912: 432 us, 298 with shared blocks; the 64 x 64 form of two blocks per CU that ran
+// there earlier took 364.  That form is still up to 8% faster where its blocks fill two rounds almost
+// exactly (726 x 3,776 x 960: 56 and 61 us; 1,190 x 1,600 x 1,216: 47 and 50), and 1.4 times slower over the
+// 90 shapes.  Below 512 rows the sums stay in four chains
 // (as many roundings as the 32-row form with four k-groups that ran there), which leaves registers for
 // at most 64 rows: 256 x 3,072 x 1,024 SwiGLU 48 -> 40, 128 x 4,096 x 1,024 15.6 -> 14.6 (us, repeated
-// calls on the same operands).
+// calls on the same operands); a round's start counts the same for all of them.
 template <int EPI>
 int launch_epi(const Params& p, hipStream_t st, int cus) {
     constexpr bool SW = EPI == GEMV_EPI_SWIGLU;
@@ -270,8 +278,10 @@ int launch_epi(const Params& p, hipStream_t st, int cus) {
         for (int b = 1; b <= max_mb; b++) {
             if (p.N % (32 * w)) continue;
             const long long blocks = (long long)((p.M + 32 * b - 1) / (32 * b)) * (p.N / (32 * w)) * p.ksplit;
-            const double rounds = (double)((blocks + cus - 1) / cus);
-            const double cost = rounds * (8.0 * b * w * (SW ? 2 : 1) * kper / 0.87 + 2500.0);
+            const double rounds = (double)((blocks + cus - 1) / cus), mfma = 8.0 * b * w * (SW ? 2 : 1) * kper;
+            double cost = rounds * (0.48e-3 * mfma + 1.0 + (p.M >= 512 ? 2.0 * b : 0.0));
+            if (p.M >= 512 && b == 1 && !SW)
+                cost = w == 2 ? rounds * (0.58e-3 * mfma + 0.75) + 1.75 : rounds * (0.495e-3 * mfma + 2.25) + 1.0;
             if (best == 0 || cost < best) {
                 best = cost;
                 mb = b;

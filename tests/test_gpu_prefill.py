@@ -214,7 +214,10 @@ def test_prefill_matches_sequential_decode_and_oracle(ctx, per_head, batch, back
                                    # 64 x 128, 96 x 64, 96 x 128, 128 x 64, 128 x 128
                                    (152, 6528, 32), (39, 8960, 64), (476, 2560, 96), (663, 576, 64),
                                    (777, 1280, 1344), (814, 1152, 32), (1185, 1664, 800), (533, 4800, 32),
-                                   (846, 3072, 96), (1411, 2368, 64), (3308, 1024, 32)])
+                                   (846, 3072, 96), (1411, 2368, 64), (3308, 1024, 32),
+                                   # (those of them that the shapes above miss, each at its smallest)
+                                   (611, 832, 576), (515, 2944, 64), (583, 1728, 640), (674, 2240, 672),
+                                   (705, 4992, 128), (587, 1728, 32), (643, 2368, 32)])
 def test_gemm_f32_vs_float64(ctx, M, N, K):
     """fp32 MFMA projection (ar_hip_gemm_f32): every tile of the launch rule, ragged M, one to many
     k-tiles of 32 (odd and even counts), all three epilogues, against float64 products of the same fp32
