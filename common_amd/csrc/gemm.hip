@@ -57,14 +57,10 @@ struct Mfma<true> {
     }
 };
 
-// up * silu(gate) for a 16-bit output: the hardware's exp2 and reciprocal (a few 2^-24 relative for the
-// gates that matter, against the 2^-9 or 2^-12 of the rounding that follows; expf and an exact division
-// are four times the instructions, and nothing overlaps the epilogue of a block that has its CU alone:
-// 2,048 x 6,144 x 2,048 SwiGLU 116 -> 98 us with these and the paired stores of gemm_dma_kernel; error
-// against 64 bits 1.7e-3 as before, all of it the bf16 output).
-__device__ inline float swiglu16(float g, float u) {
-    const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
-    return u * (g * __builtin_amdgcn_rcpf(e + 1.0f));
+// up * silu(gate), the same in every SwiGLU epilogue and in the row pass behind library products.
+__device__ inline float swiglu(float g, float u) {
+    const float sg = 1.0f / (expf(-g) + 1.0f);
+    return u * (g * sg);
 }
 
 constexpr int BN = 128, BK = 64;
@@ -220,9 +216,7 @@ __global__ __launch_bounds__(BMT * 2) void gemm_kernel(GemmParams p, int mt, int
                     float* c = Cs + (size_t)row * p.ldc + col;
                     *c = *c + v;
                 } else {
-                    const float g = v, u = acc[NW - 1][i][j][r];
-                    const float sg = 1.0f / (expf(-g) + 1.0f);
-                    const float o = u * (g * sg);
+                    const float o = swiglu(v, acc[NW - 1][i][j][r]);
                     if (F16) f16_range_check(o, p.rf);
                     p.O[(size_t)row * p.ldo + col] = M::from_float(o);
                 }
@@ -440,8 +434,8 @@ __global__ __launch_bounds__(dma::NTHR) void gemm_dma_kernel(GemmParams p, int m
 #pragma unroll
                 for (int r = 0; r < 16; r += 2) {
                     const int row = rbase + (r >> 2) * 8 + (r & 3);
-                    const float o0 = swiglu16(acc[0][i][j][r], acc[NW - 1][i][j][r]);
-                    const float o1 = swiglu16(acc[0][i][j][r + 1], acc[NW - 1][i][j][r + 1]);
+                    const float o0 = swiglu(acc[0][i][j][r], acc[NW - 1][i][j][r]);
+                    const float o1 = swiglu(acc[0][i][j][r + 1], acc[NW - 1][i][j][r + 1]);
                     if (F16) {  // (rows past M repeat row M - 1)
                         f16_range_check(o0, p.rf);
                         f16_range_check(o1, p.rf);

@@ -51,14 +51,18 @@ def test_gemm_store_bias(ctx, M, N, K):
 @pytest.mark.parametrize("M,shift", [(2048, 0), (2043, 0), (2043, 2)])
 def test_gemm_swiglu_paired_stores(ctx, M, shift):
     """The large-tile SwiGLU epilogue: two columns per store, rows past M (odd M: a pair straddles the
-    end), an output off 4-byte boundaries, and gates far past exp's range on both sides.  One bf16
-    rounding: 2^-8 of the largest value."""
+    end), an output off 4-byte boundaries, gates far past exp's range on both sides and, in one column, gates
+    whose sigmoid lies under fp32's normal range while their product does not.  Value by value: one bf16
+    rounding (2^-9, 2^-8 with its neighbour's), and the K roundings of each fp32 sum."""
     N, K = 4096, 64
     r = np.random.default_rng(M + shift)
     A = bf16(r.standard_normal((M, K)))
     W = bf16(r.standard_normal((N, K)) * 0.3)
     W[::7] = bf16(W[::7] * 100.0)
     W2 = bf16(r.standard_normal((N, K)) * 0.05)
+    A[:, 0] = 1.0
+    W[5], W2[5] = 0.0, 0.0
+    W[5, 0], W2[5, 0] = -88.0, 1e30  # silu(-88) = -5.3e-37
     guard = 64
     Od = ctx.to_device(np.full(M * N + guard, 0x7F7F, np.uint16))
     view = type("At", (), {"ptr": Od.ptr + shift})()
@@ -67,12 +71,17 @@ def test_gemm_swiglu_paired_stores(ctx, M, shift):
     ctx.synchronize()
     raw = Od.download(np.uint16, M * N + guard)
     got = (raw[shift // 2:shift // 2 + M * N].astype(np.uint32) << 16).view(np.float32).reshape(M, N)
-    assert (raw[shift // 2 + M * N:] == 0x7F7F).all()
-    g = A.astype(np.float64) @ W.astype(np.float64).T
-    u = A.astype(np.float64) @ W2.astype(np.float64).T
+    assert (raw[:shift // 2] == 0x7F7F).all() and (raw[shift // 2 + M * N:] == 0x7F7F).all()
+    A64, W64, U64 = (t.astype(np.float64) for t in (A, W, W2))
+    g, u = A64 @ W64.T, A64 @ U64.T
     with np.errstate(over="ignore"):
-        ref = u * (g / (1 + np.exp(-g)))
-    assert rel_err(got, ref) <= 2.0 ** -8
+        silu = g / (1 + np.exp(-g))
+    ref = u * silu
+    # |silu'| <= 1.1; an expf of relative error 2^-23 on top of the sums' K * 2^-24; past -88.7 expf overflows and
+    # the sigmoid is 0 (|silu| < 3e-37 there)
+    sums = K * 2.0 ** -24 * (1.1 * (np.abs(A64) @ np.abs(W64).T) * np.abs(u) + (np.abs(A64) @ np.abs(U64).T) * np.abs(silu))
+    lost = np.where(g < -88.6, np.abs(ref), 0.0)
+    assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 2 * sums + lost).all()
 
 
 def test_gemm_residual_and_swiglu(ctx):
