@@ -449,11 +449,11 @@ int decode_persistent_layer_entry(void* dst, const void* wqkv, const void* wo, c
 bool decode_persistent_supported(int wdtype, int dim, int F, int heads, int kv_heads, int hd, bool kv16);
 int launch_decode_persistent(const DecodePersistentLaunch& a, hipStream_t stream);
 size_t attention_partial_floats(int batch, int heads, int max_splits, int hd);
-// Splits for a cache of max_seq rows: about one block per CU, rows per split <= 256 (1040 for an
+// Splits for a cache of max_seq rows: about one block per CU, rows per split <= 348 (1040 for an
 // fp16 cache; one split, no combine, for caches of at most 256 rows).
 int attention_max_splits(int max_seq, int kv_heads, int batch, bool kv16);
 // The same for the stand-alone operator (one sequence, fp32 cache), in whole blocks per CU.
-int attention_whole_splits(int max_seq, int kv_heads);
+int attention_whole_splits(int max_seq, int kv_heads, int cus);
 
 // Start of a decode step (one block).  state = device {current position, prompt length, next
 // position}.  Position p = next: the token fed is the prompt token tokens[b][p] while p is inside

@@ -848,11 +848,12 @@ int attention_max_splits(int max_seq, int kv_heads, int batch, bool kv16) {
 
 // The splits of the stand-alone operator for a cache that needs more than one block per CU: whole blocks
 // per CU (32 heads, 8 KV heads, 32,768 rows: 96 splits, three blocks per CU, 55.9 us against 58.5 with the
-// 95 that cover the rows; 16,384 rows: 64, 33.8 against 36.0 with 48).  A model keeps
+// 95 that cover the rows; 16,384 rows: 64, 33.8 against 36.0 with 48; the longest ways up, 12,000 and 23,000
+// rows from 35 and 67 splits: 27.0 -> 23.2 and 39.6 -> 36.9).  A model keeps
 // attention_max_splits, measured over its batches (kMaxTile).
-int attention_whole_splits(int max_seq, int kv_heads) {
+int attention_whole_splits(int max_seq, int kv_heads, int cus) {
     const int s = attention_max_splits(max_seq, kv_heads, 1, false);
-    const int cu = 256 % kv_heads == 0 ? 256 / kv_heads : 1;  // splits of one block per CU
+    const int cu = cus % kv_heads == 0 ? cus / kv_heads : 1;  // splits of one block per CU
     const int w = (s + cu - 1) / cu * cu;
     return s > cu && w <= kMaxSplits ? w : s;
 }

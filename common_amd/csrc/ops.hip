@@ -60,7 +60,34 @@ int grow(ar_hip_ctx* ctx, void** p, size_t* have, size_t need, size_t elem) {
 }
 }  // namespace
 
+// ---- allocation-free attention -----------------------------------------------------------
+// The split partials of ar_hip_attention_decode_noalloc live in this fixed array: each GPU the
+// library runs on holds one copy (1 MiB) until the process ends.  Host code never passes the
+// array's name to a kernel: ar_ops_init looks up this device's address of it once per context,
+// with the context's device current, and launches use that address.
+constexpr size_t kNoAllocScratchFloats = (size_t)1 << 18;
+static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
+
 namespace {
+std::atomic<float*> g_scratch_addr[kMaxDevices];  // per device: its copy's address, once looked up
+
+// Partial outputs [heads][splits][hd] at the start, (max, sum) pairs [heads][splits][2] after them at a
+// 256-byte boundary: where the pairs start, and the floats of both.
+size_t noalloc_floats(int heads, int splits, int head_dim, size_t* ml_off) {
+    *ml_off = (attention_partial_floats(1, heads, splits, head_dim) + 63) / 64 * 64;
+    return *ml_off + (size_t)heads * splits * 2;
+}
+
+// Splits of the stand-alone operator: whole blocks per CU, or as few as cover the cache where only those fit
+// the fixed scratch array (both entry points, so that they give the same bits).
+int operator_splits(const ar_hip_ctx* ctx, int max_seq, int heads, int kv_heads, int head_dim) {
+    size_t off;
+    const int whole = attention_whole_splits(max_seq, kv_heads, ctx->num_cus);
+    if (noalloc_floats(heads, whole, head_dim, &off) <= kNoAllocScratchFloats) return whole;
+    const int fewest = attention_max_splits(max_seq, kv_heads, 1, false);
+    return noalloc_floats(heads, fewest, head_dim, &off) <= kNoAllocScratchFloats ? fewest : whole;
+}
+
 int attention_args(ar_hip_ctx* ctx, const float* q, const float* k, const float* v, const float* q_norm,
                    const float* k_norm, float qk_eps, int qk_norm_mode, float* k_cache, float* v_cache, int max_seq,
                    int pos, int heads, int kv_heads, int head_dim, double rope_theta, float* out, AttnLaunch* a) {
@@ -71,8 +98,8 @@ int attention_args(ar_hip_ctx* ctx, const float* q, const float* k, const float*
     a->q = q; a->k = k; a->v = v; a->qkv_stride = 0; a->q_norm = q_norm; a->k_norm = k_norm; a->qk_eps = qk_eps;
     a->per_head_norm = qk_norm_mode == AR_QK_NORM_PER_HEAD; a->kcache = k_cache; a->vcache = v_cache;
     a->max_seq = max_seq; a->pos = nullptr; a->pos_value = pos; a->heads = heads; a->kv_heads = kv_heads;
-    a->head_dim = head_dim; a->rope_theta = rope_theta; a->max_splits = attention_whole_splits(max_seq, kv_heads);
-    a->out = out; a->out_stride = heads * head_dim; a->batch = 1;
+    a->head_dim = head_dim; a->rope_theta = rope_theta; a->out = out; a->out_stride = heads * head_dim; a->batch = 1;
+    a->max_splits = operator_splits(ctx, max_seq, heads, kv_heads, head_dim);
     return AR_HIP_OK;
 }
 }  // namespace
@@ -92,18 +119,6 @@ extern "C" int ar_hip_attention_decode(ar_hip_ctx* ctx, const float* q, const fl
     a.part_o = s.part_o;
     a.part_ml = s.part_ml;
     return launch_attention_decode(a, ctx->stream);
-}
-
-// ---- allocation-free attention -----------------------------------------------------------
-// The split partials of ar_hip_attention_decode_noalloc live in this fixed array: each GPU the
-// library runs on holds one copy (1 MiB) until the process ends.  Host code never passes the
-// array's name to a kernel: ar_ops_init looks up this device's address of it once per context,
-// with the context's device current, and launches use that address.
-constexpr size_t kNoAllocScratchFloats = (size_t)1 << 18;
-static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
-
-namespace {
-std::atomic<float*> g_scratch_addr[kMaxDevices];  // per device: its copy's address, once looked up
 }
 
 int ar_ops_init(ar_hip_ctx* ctx) {
@@ -132,19 +147,10 @@ extern "C" int ar_hip_attention_decode_noalloc(ar_hip_ctx* ctx, const float* q, 
     AR_TRY(attention_args(ctx, q, k, v, q_norm, k_norm, qk_eps, qk_norm_mode, k_cache, v_cache, max_seq, pos, heads,
                           kv_heads, head_dim, rope_theta, out, &a));
     AR_CHECK_ARG(ctx->noalloc_scratch, "attention (no-alloc): scratch address of device %d unknown", ctx->device);
-    // partial outputs [heads][splits][hd] at the start, (max, sum) pairs [heads][splits][2] after
-    // them at a 256-byte boundary.  Nothing needs clearing: the combine uses only the splits this
-    // call's attention launch writes (it may load the stale slots past them, never uses them).
-    auto layout = [&](size_t* ml_off) {
-        *ml_off = (attention_partial_floats(1, heads, a.max_splits, head_dim) + 63) / 64 * 64;
-        return *ml_off + (size_t)heads * a.max_splits * 2;
-    };
-    size_t ml_off, need = layout(&ml_off);
-    if (need > kNoAllocScratchFloats) {  // as few splits as cover the cache may still fit
-        a.max_splits = attention_max_splits(max_seq, kv_heads, 1, false);
-        need = layout(&ml_off);
-    }
-    AR_CHECK_ARG(need <= kNoAllocScratchFloats,
+    // Nothing needs clearing: the combine uses only the splits this call's attention launch writes (it may
+    // load the stale slots past them, never uses them).
+    size_t ml_off;
+    AR_CHECK_ARG(noalloc_floats(heads, a.max_splits, head_dim, &ml_off) <= kNoAllocScratchFloats,
                  "attention (no-alloc): %d heads x %d splits x (%d + 2) floats of partials exceed the %zu-float "
                  "scratch (cache of %d rows); use ar_hip_attention_decode",
                  heads, a.max_splits, head_dim, kNoAllocScratchFloats, max_seq);

@@ -120,8 +120,7 @@ int ar_hip_attention_decode(ar_hip_ctx *ctx, const float *q, const float *k, con
 
 /* ar_hip_attention_decode without any allocation: no counterpart in the reference.  For callers
  * that cannot allocate device memory (code under HIP graph capture, serving loops, harnesses that
- * forbid hipMalloc).  Same arguments, kernels and results (to rounding where only fewer splits of the
- * cache fit the scratch); the split partials go to a fixed
+ * forbid hipMalloc).  Same arguments, kernels and results; the split partials go to a fixed
  * per-device scratch array of 2^18 floats (1 MiB, held by each GPU the library runs on until the
  * process ends) instead of memory the library allocates.  Rejects (AR_HIP_ERR_INVALID) shapes whose
  * partials, heads x splits x (head_dim + 2) floats, exceed it (16 heads x hd 128 caches up to
