@@ -413,10 +413,16 @@ __host__ __device__ inline void attn_split_plan(int n, int max_splits, int* nspl
 // Attention partials + (when the context is split) the combine kernel.
 int launch_attention_decode(const AttnLaunch& a, hipStream_t stream);
 
+// Words of a model's loop state on the device.  Each has one writer: the position, the prompt length and the
+// next position are the step begin's (and the host's between steps), the exchange epoch base is the
+// persistent step's, the arrival count the step begin's of several sequences, zero between steps.
+enum LoopState { kStatePos = 0, kStatePrompt, kStateNext, kStateEpoch, kStateArrived, kStateWords };
+
 // Persistent decode step (decode_persistent.hip): every layer of a batch-1 decode step in one launch
 // of one block per CU.  `layers` is a device table of layer_count entries written
 // by decode_persistent_layer_entry; `ll` holds decode_persistent_ll_words() zeroed words at first
-// use; state[0] is the position and state[3] the exchange epoch base, which every launch advances.
+// use; state[kStatePos] is the position and state[kStateEpoch] the exchange epoch base, which every
+// launch advances.
 struct DecodePersistentLaunch {
     const void* layers = nullptr;
     int layer_count = 0;
@@ -455,10 +461,11 @@ int attention_max_splits(int max_seq, int kv_heads, int batch, bool kv16);
 // The same for the stand-alone operator (one sequence, fp32 cache), in whole blocks per CU.
 int attention_whole_splits(int max_seq, int kv_heads, int cus);
 
-// Start of a decode step (one block).  state = device {current position, prompt length, next
-// position}.  Position p = next: the token fed is the prompt token tokens[b][p] while p is inside
+// Start of a decode step (one block per sequence).  state: kStateWords ints on the device (LoopState), with
+// state[kStateArrived] zero on entry and again on return.  Position p = next: the token fed is the prompt token tokens[b][p] while p is inside
 // the prompt, else the greedy choice decoded from keys[b] (the previous step's logits), which is
-// also stored at tokens[b][p]; keys are then cleared, x[b] = E[token], current = p, next = p+1.
+// also stored at tokens[b][p]; keys are then cleared, x[b] = E[token], current = p, next = p+1 (by the
+// last block to have read the position).
 // x_hi / x_lo (optional): bf16 planes of x_gain * x (bf16_planes) for the first GEMV's MFMA path;
 // ss_out (optional, [dim/16][16]): sums of squares of each 16 consecutive entries of x[b] (column b),
 // for the fragment-ordered GEMV's RMSNorm.

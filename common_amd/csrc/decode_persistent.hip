@@ -86,7 +86,7 @@ struct PParams {
     void* vcache;
     int S;
     const float2* rope_tab;  // [S][HD/2] (cos, sin)
-    int* state;        // [0] position, [3] epoch base (advanced by L at the end of every launch)
+    int* state;        // LoopState: position, epoch base (advanced by L at the end of every launch)
     uint64_t* ll;      // exchange words, two parities
     int* err;          // set to 1 when a wait timed out
     unsigned spin_limit;  // polls before a wait is abandoned
@@ -331,8 +331,8 @@ __global__ __launch_bounds__(kPT, 1) void decode_persistent_kernel(PParams p) {
     const int tid0 = threadIdx.x, b = blockIdx.x;
     int* dead = &dead_s;
     if (tid0 == 0) dead_s = 0;
-    const int pos = p.state[0];
-    const unsigned base = (unsigned)p.state[3];
+    const int pos = p.state[kStatePos];
+    const unsigned base = (unsigned)p.state[kStateEpoch];
     if (pos < 0 || pos >= p.S) {  // the host never steps past the cache; every block takes this exit
         if (b == 0 && tid0 == 0) __hip_atomic_store(p.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
@@ -1059,7 +1059,7 @@ __global__ __launch_bounds__(kPT, 1) void decode_persistent_kernel(PParams p) {
 
     // every block read the epoch base before block 0 could get here (block 0's last stage waited
     // for every block's last output), so the next launch's base can be published now
-    if (b == 0 && tid0 == 0) p.state[3] = (int)(base + (unsigned)p.L);
+    if (b == 0 && tid0 == 0) p.state[kStateEpoch] = (int)(base + (unsigned)p.L);
 }
 
 template <int DIM, int F, int H, int KV, int HD, int SMAX>
@@ -1163,7 +1163,7 @@ int launch_decode_persistent(const DecodePersistentLaunch& a, hipStream_t st) {
         AR_TRY(ar_check_range(a.kcache, cache, k, "key cache"));
         AR_TRY(ar_check_range(a.vcache, cache, k, "value cache"));
         AR_TRY(ar_check_range(a.rope_tab, (size_t)a.max_seq * (a.head_dim / 2) * sizeof(float2), k, "RoPE table"));
-        AR_TRY(ar_check_range(a.state, 4 * sizeof(int), k, "loop state"));
+        AR_TRY(ar_check_range(a.state, kStateWords * sizeof(int), k, "loop state"));
         AR_TRY(ar_check_range(a.ll, decode_persistent_ll_words(a.wdtype, a.dim, a.hidden_dim, a.heads, a.kv_heads,
                                                                a.head_dim) * 8, k, "exchange words"));
         AR_TRY(ar_check_range(a.err, sizeof(int), k, "error flag"));

@@ -16,8 +16,8 @@ __device__ inline bool better(float v1, int i1, float v2, int i2) {
 // Start of a decode step, one block per sequence: picks the token fed at position p (the prompt token,
 // or the greedy choice of the previous step decoded from the packed argmax keys), clears the sequence's
 // keys, copies the embedding row and, in the last block to have read the position, publishes p as the
-// step's position and p + 1 as the next (state[3] counts the blocks that have read it; zero between
-// steps).  A chain of memory round trips (position, keys, embedding row), the same for every sequence,
+// step's position and p + 1 as the next (state[kStateArrived] counts the blocks that have read it; zero
+// between steps).  A chain of memory round trips (position, keys, embedding row), the same for every sequence,
 // so they run side by side: 8 sequences of the 4B shape 6.7 us, 30 us with one block walking
 // them.
 // AutoregressiveModel.next + embedding copy (engine/ml/.../AutoregressiveModel.java:295-308,430).
@@ -29,8 +29,8 @@ __global__ __launch_bounds__(1024) void step_begin_kernel(const WT* table, int d
     __shared__ int tok_s;
     __shared__ unsigned long long red[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x;
-    const int p = state[2];
-    const int plen = state[1];
+    const int p = state[kStateNext];
+    const int plen = state[kStatePrompt];
     unsigned long long k = 0ull;
     if (tid < kArgmaxSlots) {
         k = keys[(size_t)b * kArgmaxSlots + tid];
@@ -59,12 +59,13 @@ __global__ __launch_bounds__(1024) void step_begin_kernel(const WT* table, int d
     if (tid == 0) {
         bool last = gridDim.x == 1;
         if (!last) {
-            last = __hip_atomic_fetch_add(state + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
-            if (last) __hip_atomic_store(state + 3, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            int* const arrived = state + kStateArrived;
+            last = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+            if (last) __hip_atomic_store(arrived, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (last) {
-            state[0] = p;
-            state[2] = p + 1;
+            state[kStatePos] = p;
+            state[kStateNext] = p + 1;
         }
     }
     const WT* row = table + (size_t)tok_s * dim;
@@ -193,7 +194,7 @@ int launch_step_begin(const void* table, int wdtype, int dim, int vocab, int* to
         AR_TRY(ar_check_range(table, (size_t)vocab * dim * wb, k, "embedding table"));
         AR_TRY(ar_check_range(tokens, (size_t)batch * token_stride * 4, k, "token rows"));
         AR_TRY(ar_check_range(keys, (size_t)batch * kArgmaxSlots * 8, k, "argmax keys"));
-        AR_TRY(ar_check_range(state, 4 * sizeof(int), k, "loop state"));
+        AR_TRY(ar_check_range(state, kStateWords * sizeof(int), k, "loop state"));
         AR_TRY(ar_check_range(x, (B1 * x_stride + dim) * 4, k, "residual rows"));
         AR_TRY(ar_check_range(x_hi, (B1 * x_stride + dim) * 2, k, "hi plane"));
         AR_TRY(ar_check_range(x_lo, (B1 * x_stride + dim) * 2, k, "lo plane"));

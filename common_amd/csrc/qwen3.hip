@@ -102,7 +102,7 @@ struct ar_qwen3 {
     void* smp_work = nullptr;
     float2* rope_tab = nullptr;             // [S][hd/2] (cos, sin), computed in double on the host
     int* tokens = nullptr;    // [B][S+1]
-    int* state = nullptr;     // {current position, prompt length, next position, step-begin blocks arrived}
+    int* state = nullptr;     // kStateWords ints (LoopState)
     float* staging = nullptr; // fp32 upload staging for dtype conversion
     size_t staging_floats = 0;
     int max_splits = 1;
@@ -634,7 +634,7 @@ extern "C" int ar_hip_qwen3_create(ar_hip_ctx* ctx, const ar_qwen3_cfg* cfg, ar_
     }
     ALLOC(rope_tab, (size_t)m->S * (c.head_size / 2) * sizeof(float2));
     ALLOC(tokens, B * (m->S + 1) * 4);
-    ALLOC(state, 64);
+    ALLOC(state, 64);  // (kStateWords ints)
     ALLOC(staging, m->staging_floats * 4);
 #undef ALLOC
     {
@@ -769,7 +769,7 @@ static int recompute_timed_out(ar_qwen3* m, int start, int n, bool store_logits)
     for (int i = 0; i < n && rc == AR_HIP_OK; i++) rc = run_step(m, store_logits);
     m->pk_suspended = false;
     AR_TRY(rc);
-    AR_HIP_TRY(hipMemcpyAsync(m->state + 1, &m->prompt_len, sizeof(int), hipMemcpyHostToDevice, st));
+    AR_HIP_TRY(hipMemcpyAsync(m->state + kStatePrompt, &m->prompt_len, sizeof(int), hipMemcpyHostToDevice, st));
     AR_HIP_TRY(hipStreamSynchronize(st));
     m->pk_on = false;
     m->pk_recomputed += n;
@@ -869,7 +869,8 @@ extern "C" int ar_hip_qwen3_set_prompt(ar_qwen3* m, int seq, const int32_t* ids,
                                   m->ctx->stream));
     m->prompt_len = n;
     m->prompt_set[seq] = 1;
-    AR_HIP_TRY(hipMemcpyAsync(m->state + 1, &m->prompt_len, sizeof(int), hipMemcpyHostToDevice, m->ctx->stream));
+    AR_HIP_TRY(hipMemcpyAsync(m->state + kStatePrompt, &m->prompt_len, sizeof(int), hipMemcpyHostToDevice,
+                              m->ctx->stream));
     AR_HIP_TRY(hipStreamSynchronize(m->ctx->stream));
     return AR_HIP_OK;
 }
@@ -1255,8 +1256,8 @@ static int prefill_finish(ar_qwen3* m, int T, int pending, float* logits_out) {
     h.y = (logits_out || sampling) ? m->logits : nullptr;
     h.y_stride = c.vocab_size; h.epilogue = GEMV_EPI_ARGMAX; h.keys = m->am_keys;
     AR_TRY(launch_gemv(h, st));
-    const int state[3] = {T - 1, T, T};
-    AR_HIP_TRY(hipMemcpyAsync(m->state, state, sizeof(state), hipMemcpyHostToDevice, st));
+    const int loop[3] = {T - 1, T, T};
+    AR_HIP_TRY(hipMemcpyAsync(m->state, loop, sizeof(loop), hipMemcpyHostToDevice, st));
     if (sampling) AR_TRY(enqueue_sample(m));  // the first generated token
     if (logits_out)
         AR_HIP_TRY(hipMemcpyAsync(logits_out, m->logits, (size_t)B * c.vocab_size * 4, hipMemcpyDeviceToHost, st));

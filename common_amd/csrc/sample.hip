@@ -710,7 +710,7 @@ __global__ __launch_bounds__(kThreads) void smp_draw_kernel(Args a) {
     const int b = blockIdx.x, t = threadIdx.x, lane = t & 63;
     // The model draws only when the next step feeds a sampled token (past the prompt), as
     // AutoregressiveModel.next applies its sample function (AutoregressiveModel.java:295-308).
-    if (a.state && a.state[2] < a.state[1]) return;
+    if (a.state && a.state[kStateNext] < a.state[kStatePrompt]) return;
     const double D = a.topp ? 1.0 : denom(a, b);  // (the nucleus search left probabilities in buf)
     const Nucleus n = a.topp ? finish_search(a, b, L, ured) : Nucleus{false, 0, 0};
     if (t < 64) {

@@ -2,6 +2,7 @@
 and reports errors through the documented channel.  No compute call needs a GPU here."""
 import ctypes
 import os
+import re
 import subprocess
 
 import pytest
@@ -119,3 +120,18 @@ def test_kv_dtype_default_from_environment(monkeypatch):
     monkeypatch.setenv("AR_HIP_KV_DTYPE", "int4")
     with pytest.raises(ValueError):
         C.Qwen3Config(dim=64, hidden_dim=64, layer_count=1, head_count=1, kv_head_count=1, vocab_size=8, seq_len=4)
+
+
+def test_loop_state_words_are_named_and_have_one_owner_each():
+    """The loop state's words are shared between kernels of several files: they go by the names of LoopState,
+    which no two words share, and the counter of the step begin's blocks is not the persistent step's epoch."""
+    csrc = os.path.join(os.path.dirname(_native.__file__), "csrc")
+    text = {f: open(os.path.join(csrc, f)).read() for f in sorted(os.listdir(csrc)) if f.endswith((".hip", ".h"))}
+    bare = [f"{f}: {m.group(0)}" for f, t in text.items()
+            for m in re.finditer(r"\bstate\s*(?:\[\s*\d+\s*\]|\+\s*\d+)", t)]
+    assert not bare, bare
+    words = re.search(r"enum LoopState \{ (.*?) \};", text["ar_hip_internal.h"]).group(1)
+    names = [w.split("=")[0].strip() for w in words.split(",")]
+    assert names == ["kStatePos", "kStatePrompt", "kStateNext", "kStateEpoch", "kStateArrived", "kStateWords"]
+    users = lambda name: {f for f, t in text.items() if f.endswith(".hip") and name in t}  # noqa: E731
+    assert users("kStateArrived") == {"misc.hip"} and users("kStateEpoch") == {"decode_persistent.hip"}
