@@ -12,7 +12,9 @@ Checked here:
 * the Qwen3-0.6B layer shape with bf16 weights at batch 3 (sequences 3..7 of the MFMA columns
   unused, most tiles shared by several wavefronts) against the FP32 oracle run on the same bf16-rounded
   weights: logits within 2e-2 and the greedy tokens equal where the reference's top-2 margin is
-  above that tolerance (the bar of the other bf16 workload tests).
+  above that tolerance (the bar of the other bf16 workload tests);
+* widths whose row-major products hold 13 to 16 k-steps a wavefront (the 8B shape's 4,096 among them), three
+  sequences, with and without the fragment GEMVs, against the FP64 oracle.
 """
 import dataclasses
 
@@ -92,3 +94,27 @@ def test_fragment_gemv_batch3_vs_oracle(ctx):
             compared += 1
         print(f"  seq {b}: {compared} steps equal to the oracle", flush=True)
         assert compared >= n + 2
+
+
+@pytest.mark.parametrize("dim", [3328, 3616, 4096])
+def test_wide_row_major_products_vs_oracle(ctx, dim):
+    """QKV (6,144 rows) and the head (4,352) read operand planes and the RMSNorm's raw input in the packed
+    row-major form; with the fragment GEMVs off so does the 4,096-wide O product where the model is as wide.
+    Two bf16 planes carry 16 bits of an input (2^-17 relative), through four products and a residual stream:
+    1e-4."""
+    cfg = C.Qwen3Config(dim=dim, hidden_dim=512, layer_count=1, head_count=32, kv_head_count=8, vocab_size=4352,
+                        seq_len=16, head_size=128, max_batch=3, weight_dtype=C.DTYPE_BF16, kv_dtype=C.DTYPE_F32)
+    sd = synthetic.state_dict(cfg, seed=dim)
+    prompts = synthetic.prompt_ids(3, cfg.vocab_size, seed=35, batch=3)
+    with Qwen3(cfg, sd, ctx) as m:
+        runs = []
+        for frag in (True, False):
+            m.model.use_fragment_gemv(frag)
+            runs.append(_decode(m.model, prompts, 1))
+    for b in range(3):
+        ref = oracle.OracleQwen3(dataclasses.replace(cfg, max_batch=1), sd, precision="fp64")
+        _, rl = ref.generate(prompts[b], 1)
+        ref.close()
+        for _, lgs in runs:
+            for s in range(len(prompts[b])):
+                assert rel_err(lgs[b, s], rl[s]) <= 1e-4, (b, s, rel_err(lgs[b, s], rl[s]))

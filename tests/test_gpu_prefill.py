@@ -219,12 +219,12 @@ def test_prefill_matches_sequential_decode_and_oracle(ctx, per_head, batch, back
 @pytest.mark.parametrize("M,N,K", [(1, 64, 32), (16, 512, 256), (33, 64, 96), (40, 128, 768), (100, 768, 1024),
                                    (128, 4096, 1024), (600, 1024, 3072), (520, 128, 160),
                                    # the tiles of the launch rule on 256 CUs, ragged M: below 512 rows
-                                   # 32 x 128, 64 x 64, 64 x 128; from 512 rows 32 x 64, 32 x 128, 64 x 64,
-                                   # 64 x 128, 96 x 64, 96 x 128, 128 x 64, 128 x 128
+                                   # 32 x 128, 64 x 64, 64 x 128; from 512 rows 32 x 64, 32 x 128 (a CU
+                                   # shared), 64 x 128, 96 x 128, SwiGLU's 64, 96 and 128 x 64
                                    (152, 6528, 32), (39, 8960, 64), (476, 2560, 96), (663, 576, 64),
                                    (777, 1280, 1344), (814, 1152, 32), (1185, 1664, 800), (533, 4800, 32),
                                    (846, 3072, 96), (1411, 2368, 64), (3308, 1024, 32),
-                                   # (those of them that the shapes above miss, each at its smallest)
+                                   # 64 x 64, 64 x 128, 96 x 64, 128 x 64, 128 x 128; SwiGLU's 96 and 128 x 64
                                    (611, 832, 576), (515, 2944, 64), (583, 1728, 640), (674, 2240, 672),
                                    (705, 4992, 128), (587, 1728, 32), (643, 2368, 32)])
 def test_gemm_f32_vs_float64(ctx, M, N, K):
