@@ -63,6 +63,21 @@ __device__ inline float swiglu(float g, float u) {
     return u * (g * sg);
 }
 
+// The same for |gate| <= 87, where no step leaves the normal range: e^-g as 2^t e^d, t = -g log2(e) rounded,
+// d = -g - t ln 2 its error, and g / (1 + e^-g) from the reciprocal with one correction of the quotient.
+// Half of swiglu's instructions, for the epilogue of a block that has its CU alone (nothing overlaps it):
+// 2,048 x 6,144 x 2,048 103 us, with swiglu 107, with the bare exp2 and reciprocal 98.  Distance from 64 bits in
+// units of 2^-24, rms over 2 million gates: 0.68 within 1 of 0, 0.72 within 10, 0.75 from -30 to -5, 0.74 from -87 to
+// -30 (largest 4); swiglu 0.80, 0.77, 0.76, 0.75 (3.4); the bare forms 0.83, 2.0, 9.5, 27, and 0 instead of some
+// 1e-37 under -87.3, where the reciprocal would be subnormal.
+__device__ inline float swiglu_87(float g, float u) {
+    const float t = g * -1.44269502f;
+    const float d = fmaf(t, 1.90465421e-9f, fmaf(t, -0.693147182f, -g));  // ln 2 = 0.693147182 - 1.904654e-9
+    const float e = __builtin_amdgcn_exp2f(t), den = fmaf(e, d, e) + 1.0f;
+    const float r = __builtin_amdgcn_rcpf(den), q = g * r;
+    return u * fmaf(fmaf(-den, q, g), r, q);
+}
+
 constexpr int BN = 128, BK = 64;
 constexpr int LDS_STRIDE = BK + 8;  // bf16 elements per LDS row
 
@@ -431,11 +446,20 @@ __global__ __launch_bounds__(dma::NTHR) void gemm_dma_kernel(GemmParams p, int m
 #pragma unroll
             for (int j = 0; j < FN; j++) {
                 const int col = n0 + wn * WN + j * 32 + (lane & 31);
+                float big = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) big = fmaxf(big, fabsf(acc[0][i][j][r]));
+                if (__ballot(big > 87.f)) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[0][i][j][r] = swiglu(acc[0][i][j][r], acc[NW - 1][i][j][r]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[0][i][j][r] = swiglu_87(acc[0][i][j][r], acc[NW - 1][i][j][r]);
+                }
 #pragma unroll
                 for (int r = 0; r < 16; r += 2) {
                     const int row = rbase + (r >> 2) * 8 + (r & 3);
-                    const float o0 = swiglu(acc[0][i][j][r], acc[NW - 1][i][j][r]);
-                    const float o1 = swiglu(acc[0][i][j][r + 1], acc[NW - 1][i][j][r + 1]);
+                    const float o0 = acc[0][i][j][r], o1 = acc[0][i][j][r + 1];
                     if (F16) {  // (rows past M repeat row M - 1)
                         f16_range_check(o0, p.rf);
                         f16_range_check(o1, p.rf);

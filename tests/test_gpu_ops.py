@@ -186,7 +186,7 @@ def test_attention_c2(ctx, per_head):
     (8, 8, 128, 100, 63), (16, 2, 128, 700, 699), (8, 8, 128, 1000, 999), (4, 2, 64, 600, 599),
     (8, 1, 128, 4096, 4000),
     # more than 32 splits: the merge in four groups of threads, with few, some and all splits live, and
-    # (90,000 rows: 512 splits, 500 of them live) more splits than the 256 threads of a merge block
+    # (90,000 rows: 512 splits) more splits than the 256 threads of a merge block
     (4, 2, 64, 2100, 20), (4, 2, 128, 2100, 1500), (4, 1, 64, 20000, 19999), (16, 8, 128, 16000, 15000),
     (12, 12, 64, 12000, 11999), (4, 1, 64, 90000, 87900)])
 def test_attention_edges(ctx, heads, kv, hd, max_seq, pos):

@@ -77,11 +77,15 @@ def test_gemm_swiglu_paired_stores(ctx, M, shift):
     with np.errstate(over="ignore"):
         silu = g / (1 + np.exp(-g))
     ref = u * silu
-    # |silu'| <= 1.1; an expf of relative error 2^-23 on top of the sums' K * 2^-24; past -88.7 expf overflows and
-    # the sigmoid is 0 (|silu| < 3e-37 there)
-    sums = K * 2.0 ** -24 * (1.1 * (np.abs(A64) @ np.abs(W64).T) * np.abs(u) + (np.abs(A64) @ np.abs(U64).T) * np.abs(silu))
-    lost = np.where(g < -88.6, np.abs(ref), 0.0)
-    assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 2 * sums + lost).all()
+    # |silu'| <= 1.1, and (1 + |g|) e^g on the left; the sums' K * 2^-24, twice for the silu's own roundings; past
+    # -88.7 expf overflows and the sigmoid is 0 (|silu| < 3e-37 there)
+    slope = np.minimum(1.1, (1 + np.abs(g)) * np.exp(np.minimum(g, 0.0)))
+    sums = K * 2.0 ** -24 * (slope * (np.abs(A64) @ np.abs(W64).T) * np.abs(u) +
+                             (np.abs(A64) @ np.abs(U64).T) * np.abs(silu))
+    # (subnormal sigmoids, from -87.3 on, keep fewer bits: 2^-5; subnormal results have no relative bound)
+    lost = np.where(g < -88.6, 1.0, np.where(g < -87.3, 2.0 ** -5, 0.0)) * np.abs(ref) + 2.0 ** -126
+    bad = np.argwhere(~(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 2 * sums + lost))
+    assert len(bad) == 0, (len(bad), [(m, n, g[m, n], u[m, n], got[m, n], ref[m, n]) for m, n in bad[:5]])
 
 
 def test_gemm_residual_and_swiglu(ctx):
