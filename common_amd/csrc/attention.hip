@@ -594,8 +594,8 @@ int pick_g(const AttnLaunch& a, hipStream_t s) {
 // of two accumulators of its own and added to the sum by the vector units while the next one runs: one
 // accumulator for a whole sum (128 dims, a quarter of the keys) was 1.5 to 1.9 times as far from 64 bits as
 // this and as the vector form (3.1e-7, 1.9e-7 and 1.8e-7 at 100 rows), for 98 instead of 109 us.
-// 0.6B shape (16 heads, 8 KV heads, hd 128), 1,531 rows: 109 us (88 TFLOP/s of the causal half, 58% of the
-// matrix rate; the rest is the uneven end of the causal blocks and each block's start and merge) against
+// 0.6B shape (16 heads, 8 KV heads, hd 128), 1,531 rows: 109 us (88 TFLOP/s of the causal half; MFMA busy
+// 53%, the rest is the uneven end of the causal blocks and each block's start and merge) against
 // 382 us for one block per (row, KV head) on the vector units, where each row reads its whole context; 128
 // rows 11.1 against 11.4 us.
 struct PrefillAttnF32 {

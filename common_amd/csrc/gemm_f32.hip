@@ -316,6 +316,8 @@ int launch_epi(const Params& p, hipStream_t st, int cus) {
 
 }  // namespace
 
+// k-slices of a residual product whose partials the next RMSNorm folds: as many as fill the CUs with 32-row
+// (from 512 rows 64-row) x 64 tiles.  The launch then takes the tile for the slices.
 int gemm_f32_ksplit(int M, int N, int K, int cus) {
     const int bm = M >= 512 ? 64 : 32;
     const long long tiles = (long long)((M + bm - 1) / bm) * (N / 64);
